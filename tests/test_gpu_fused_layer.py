@@ -87,6 +87,22 @@ def test_rms_norm_vs_oracle(ops, dtype):
             assert off <= max(1, y.numel() // 100), f"{dtype} m={m} k={k}: {off} elements not rounded"
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("k", [8, 504, 512, 520, 1024, 1032, 2048, 2056, 4096, 4104, 8192, 8200])
+def test_rms_norm_row_lengths(ops, dtype, k):
+    """Every vector-count branch of the row kernel and the lengths around it, strided rows included, held to
+    the bound of test_rms_norm_vs_oracle."""
+    g = torch.Generator(device="cuda").manual_seed(k)
+    x = (torch.randn(5, k + 8, device="cuda", generator=g) * 2).to(dtype)[:, :k]
+    w = (1 + 0.2 * torch.randn(k, device="cuda", generator=g)).to(dtype)
+    y = ops.rms_norm(x, w, 1e-6)
+    ref = O.rms_norm(_bits(x), _bits(w), 1e-6, _TD[dtype])
+    want = _round(ref, dtype).double().numpy()
+    err = np.abs(y.double().cpu().numpy() - want)
+    assert (err <= _ulp(want, dtype)).all()
+    assert (err > 0).mean() <= 0.01
+
+
 def test_rms_norm_golden(ops):
     z = np.load(os.path.join(GOLDEN, "rms_norm.npz"))
     eps = float(z["eps"])

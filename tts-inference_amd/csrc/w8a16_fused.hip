@@ -9,7 +9,7 @@
 //
 //  * rms_norm_*_kernel: RMSNorm on its own (qtts/layers/norm.py:50-76): fp32 sum of
 //    squares, inv = 1 / sqrt(sum / K + eps) correctly rounded, (x * inv) * w rounded
-//    to the activation dtype.  One wave a row.
+//    to the activation dtype.
 //  * silu_mul_*_kernel: `F.silu(gate) * up` in one pass with torch's two roundings
 //    (common.h: silu_mul).
 //  * residual_add_kernel: y = residual + t, for calls whose GEMM cannot add it (the
@@ -52,44 +52,62 @@ __global__ __launch_bounds__(kEltThreads) void silu_mul_kernel(const XT* __restr
     h[r * ldh + c] = from_f32<XT>(silu_mul<XT>(to_f32(gu[r * ld + c]), to_f32(gu[r * ld + k + c])));
 }
 
-// RMSNorm, one wave a row, 4 rows a workgroup.  Vector form: 16-bit rows, 16-byte
-// aligned, k % 8 == 0; lane l owns elements 512 v + 8 l .. + 7.  The row is read
-// twice (the second time from cache): once for the sum, once to scale it.
-constexpr int kNormRowsPerBlock = 4;
-
-template <typename XT>
-__global__ __launch_bounds__(64 * kNormRowsPerBlock) void rms_norm_vec_kernel(const XT* __restrict__ x, int64_t ldx,
-                                                                             const XT* __restrict__ w, int k, float eps,
-                                                                             XT* __restrict__ y, int64_t ldy, int m) {
-  const int lane = threadIdx.x & 63;
-  const int64_t row = (int64_t)blockIdx.x * kNormRowsPerBlock + (threadIdx.x >> 6);
-  if (row >= m) return;
+// RMSNorm, vector form (16-bit rows, 16-byte aligned, k % 8 == 0, k <= 8192): one row a workgroup of T
+// threads, thread t holding vectors t, t + T, ... of the row and of the weight in registers, so a row costs
+// one memory round trip and one LDS exchange.  Bound by that latency at the decode and prompt sizes (32 rows
+// of 2048 are 256 KB in and out): one wave a row that read it twice in a loop took 5.1 us there under a trace
+// and 5.9 at 1003 rows; a 12-layer talker step of 32 rows went from 579.7 to 524.5 us (2.3 us a norm), the
+// predictor's 8-stream frame from 2750 to 2645.
+template <typename XT, int T, int V>
+__global__ __launch_bounds__(T) void rms_norm_vec_kernel(const XT* __restrict__ x, int64_t ldx,
+                                                         const XT* __restrict__ w, int k, float eps,
+                                                         XT* __restrict__ y, int64_t ldy) {
+  __shared__ float part[T / 64];
+  const int tid = threadIdx.x, nv = k >> 3;
+  const int64_t row = blockIdx.x;
   const XT* xr = x + row * ldx;
+  i32x4_t v[V], wv[V];
+#pragma unroll
+  for (int j = 0; j < V; ++j) v[j] = *(const i32x4_t*)(xr + 8 * min(tid + T * j, nv - 1));  // clamped: in the row
+#pragma unroll
+  for (int j = 0; j < V; ++j) wv[j] = *(const i32x4_t*)(w + 8 * min(tid + T * j, nv - 1));
   float ss = 0.0f;
-  for (int e0 = 8 * lane; e0 < k; e0 += 512) {
-    const i32x4_t v = *(const i32x4_t*)(xr + e0);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const float a = to_f32(XT{(uint16_t)v[i]}), b = to_f32(XT{(uint16_t)((uint32_t)v[i] >> 16)});
-      ss = __builtin_fmaf(a, a, ss);
-      ss = __builtin_fmaf(b, b, ss);
-    }
+  for (int j = 0; j < V; ++j)
+    if (tid + T * j < nv)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float a = to_f32(XT{(uint16_t)v[j][i]}), b = to_f32(XT{(uint16_t)((uint32_t)v[j][i] >> 16)});
+        ss = __builtin_fmaf(a, a, ss);
+        ss = __builtin_fmaf(b, b, ss);
+      }
+  ss = wave_sum_rows(ss);
+  if constexpr (T > 64) {
+    if ((tid & 63) == 0) part[tid >> 6] = ss;
+    __syncthreads();
+    ss = part[0];
+#pragma unroll
+    for (int i = 1; i < T / 64; ++i) ss += part[i];
   }
-  ss = wave_sum(ss);
   const float inv = 1.0f / __builtin_sqrtf(ss / (float)k + eps);
-  for (int e0 = 8 * lane; e0 < k; e0 += 512) {
-    const i32x4_t v = *(const i32x4_t*)(xr + e0), wv = *(const i32x4_t*)(w + e0);
-    i32x4_t o;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const uint32_t p = (uint32_t)v[i], q = (uint32_t)wv[i];
-      const float h0 = (to_f32(XT{(uint16_t)p}) * inv) * to_f32(XT{(uint16_t)q});
-      const float h1 = (to_f32(XT{(uint16_t)(p >> 16)}) * inv) * to_f32(XT{(uint16_t)(q >> 16)});
-      o[i] = (int)pack2_f32<XT>(h0, h1);
+  for (int j = 0; j < V; ++j)
+    if (tid + T * j < nv) {
+      i32x4_t o;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const uint32_t p = (uint32_t)v[j][i], q = (uint32_t)wv[j][i];
+        const float h0 = (to_f32(XT{(uint16_t)p}) * inv) * to_f32(XT{(uint16_t)q});
+        const float h1 = (to_f32(XT{(uint16_t)(p >> 16)}) * inv) * to_f32(XT{(uint16_t)(q >> 16)});
+        o[i] = (int)pack2_f32<XT>(h0, h1);
+      }
+      *(i32x4_t*)(y + row * ldy + 8 * (tid + T * j)) = o;
     }
-    *(i32x4_t*)(y + row * ldy + e0) = o;
-  }
 }
+
+// The other rows (fp32, ragged or unaligned, longer): one wave a row, 4 rows a workgroup, the row read
+// twice (the second time from cache).
+constexpr int kNormRowsPerBlock = 4;
 
 template <typename XT>
 __global__ __launch_bounds__(64 * kNormRowsPerBlock) void rms_norm_kernel(const XT* __restrict__ x, int64_t ldx,
@@ -169,14 +187,32 @@ int qtts_launch_silu_mul(const void* gu, int x_dtype, int64_t m, int64_t k, int6
 
 int qtts_launch_rms_norm(const void* x, int x_dtype, int64_t m, int64_t k, int64_t ldx, const void* w, float eps,
                          void* y, int64_t ldy, hipStream_t st) {
-  const bool vec = x_dtype != QTTS_F32 && k % 8 == 0 && (uintptr_t)x % 16 == 0 && (uintptr_t)w % 16 == 0 &&
-                   (uintptr_t)y % 16 == 0 && ldx % 8 == 0 && ldy % 8 == 0;
+  const int64_t nv = k / 8;
+  const bool vec = x_dtype != QTTS_F32 && k % 8 == 0 && k > 0 && nv <= 1024 && m <= (1 << 22) && (uintptr_t)x % 16 == 0 &&
+                   (uintptr_t)w % 16 == 0 && (uintptr_t)y % 16 == 0 && ldx % 8 == 0 && ldy % 8 == 0;
+  if (vec) {
+    // the fewest threads (64 to 256) that hold the row in one vector each, then more vectors a thread
+#define QTTS_NORM_VEC(T, TH, V)                                                                             \
+  qtts::launch(&rms_norm_vec_kernel<T, TH, V>, dim3((unsigned)m), dim3(TH), 0, st, (const T*)x, ldx, (const T*)w, \
+               (int)k, eps, (T*)y, ldy)
+#define QTTS_NORM_T(T)                             \
+  do {                                             \
+    if (nv <= 64) QTTS_NORM_VEC(T, 64, 1);         \
+    else if (nv <= 128) QTTS_NORM_VEC(T, 128, 1);  \
+    else if (nv <= 256) QTTS_NORM_VEC(T, 256, 1);  \
+    else if (nv <= 512) QTTS_NORM_VEC(T, 256, 2);  \
+    else QTTS_NORM_VEC(T, 256, 4);                 \
+  } while (0)
+    if (x_dtype == QTTS_BF16) QTTS_NORM_T(bf16_t);
+    else QTTS_NORM_T(f16_t);
+#undef QTTS_NORM_T
+#undef QTTS_NORM_VEC
+    return qtts_check_launch("rms_norm");
+  }
   const dim3 grid((unsigned)((m + kNormRowsPerBlock - 1) / kNormRowsPerBlock)), block(64 * kNormRowsPerBlock);
 #define QTTS_NORM(KER, T) \
   qtts::launch(&KER<T>, grid, block, 0, st, (const T*)x, ldx, (const T*)w, (int)k, eps, (T*)y, ldy, (int)m)
-  if (vec && x_dtype == QTTS_BF16) QTTS_NORM(rms_norm_vec_kernel, bf16_t);
-  else if (vec) QTTS_NORM(rms_norm_vec_kernel, f16_t);
-  else if (x_dtype == QTTS_BF16) QTTS_NORM(rms_norm_kernel, bf16_t);
+  if (x_dtype == QTTS_BF16) QTTS_NORM(rms_norm_kernel, bf16_t);
   else if (x_dtype == QTTS_F16) QTTS_NORM(rms_norm_kernel, f16_t);
   else QTTS_NORM(rms_norm_kernel, float);
 #undef QTTS_NORM
