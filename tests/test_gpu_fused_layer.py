@@ -100,7 +100,7 @@ def test_rms_norm_row_lengths(ops, dtype, k):
     want = _round(ref, dtype).double().numpy()
     err = np.abs(y.double().cpu().numpy() - want)
     assert (err <= _ulp(want, dtype)).all()
-    assert (err > 0).mean() <= 0.01
+    assert int((err > 0).sum()) <= max(1, y.numel() // 100)
 
 
 def test_rms_norm_golden(ops):

@@ -9,17 +9,18 @@
 //
 // Same pipeline as the W8A16 tile kernel (tile.hip): 4 waves (8, two a SIMD, on the
 // larger tiles) own a BM x BN tile and walk K through a P-deep LDS ring filled by
-// direct global -> LDS loads, one barrier per stage.  A stage is 128 K columns, and
-// every load writes one 1 KiB half of the stage's MFMA fragments in lane order (lane l:
-// row l % 16 of a 16-row block, 16 bytes at stage column Kind::col(l / 16, h)):
+// direct global -> LDS loads, one barrier per stage.  A stage is 128 K columns.  A load
+// writes 1 KiB: eight activation rows of 128 bytes, their pieces swizzled (pipe.h: swizzle8),
+// or one half of a strip's MFMA fragment in lane order (lane l: row l % 16 of the strip,
+// 16 bytes at stage column Kind::col(l / 16, h)); operand half h of lane l is
+// the 16 bytes at column Kind::col(l / 16, h) of row l % 16:
 //   * fp8: the two halves are the 32-byte operand of one
 //     v_mfma_scale_f32_16x16x128_f8f6f4 (unit block scales); col = 32 g + 16 h, the
 //     QTTS_STRIP_FP8 block's lane order;
 //   * int8: each half is the 16-byte operand of one v_mfma_i32_16x16x64_i8 over one
 //     64-column chunk; col = 64 h + 16 g, two consecutive QTTS_STRIP_INT8 blocks.
 // With strip weights a weight half is 1 KiB of contiguous memory; with row-major
-// weights (int8 only) it is gathered like an activation half, 64 contiguous bytes a
-// row.  Of NW waves, wave w owns columns [n0 + w BN/NW, n0 + (w+1) BN/NW) for all BM rows.
+// weights (int8 only) it is gathered in lane order, 64 contiguous bytes a row.  Of NW waves, wave w owns columns [n0 + w BN/NW, n0 + (w+1) BN/NW) for all BM rows.
 #pragma once
 
 #include <algorithm>
@@ -137,9 +138,9 @@ __global__ __launch_bounds__(NW * 64) void w8a8_pipe_kernel(
   for (int j = 0; j < FPW; ++j) {
     const int f = wave * FPW + j;
     if (f < XF) {
-      const int mb = f >> 1, h = f & 1;
-      const int m = min(m0 + mb * 16 + c16, M - 1);
-      src[j] = qx + (int64_t)m * ldqx + (int64_t)kc0 * 128 + Kind::col(g, h);
+      const int row = 8 * f + (lane >> 3);
+      const int m = min(m0 + row, M - 1);
+      src[j] = qx + (int64_t)m * ldqx + (int64_t)kc0 * 128 + 16 * swizzle8(row, lane & 7);
       stride[j] = 128;
     } else {
       const int sb = (f - XF) >> 1, h = (f - XF) & 1;
@@ -168,11 +169,13 @@ __global__ __launch_bounds__(NW * 64) void w8a8_pipe_kernel(
 
   // A stage's operands: every activation half of the tile, and this wave's weight halves.
   struct Ops { i32x4_t x0[MB], x1[MB], w0[NB], w1[NB]; };
+  const int xoff0 = c16 * 128 + 16 * swizzle8(c16, Kind::col(g, 0) >> 4);
+  const int xoff1 = c16 * 128 + 16 * swizzle8(c16, Kind::col(g, 1) >> 4);
   auto read = [&](Ops& o, const uint8_t* stage) __attribute__((always_inline)) {
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb) {
-      o.x0[mb] = *(const i32x4_t*)(stage + (2 * mb) * 1024 + lane * 16);
-      o.x1[mb] = *(const i32x4_t*)(stage + (2 * mb + 1) * 1024 + lane * 16);
+      o.x0[mb] = *(const i32x4_t*)(stage + mb * 2048 + xoff0);
+      o.x1[mb] = *(const i32x4_t*)(stage + mb * 2048 + xoff1);
     }
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) {

@@ -12,12 +12,14 @@
 // read-ahead (PF, 3 stages or more) a wave reads the next stage's operands from LDS
 // into a second register set while the MFMAs of the current one run, so no LDS
 // latency sits between a stage's barrier and its first MFMA; P-2 stages of global
-// loads are then in flight.  Every load writes one 1 KiB MFMA fragment in lane order:
-//   * activation fragment (m-block mb, half h): lane l carries
-//     x[m0 + 16 mb + l % 16][k + 16 (l / 16) + 8 h .. + 7]  (8 bf16);
+// loads are then in flight.  A load writes 1 KiB:
+//   * activations: eight rows of the stage's 64 columns, 128 bytes each, their 16-byte pieces
+//     swizzled (pipe.h: swizzle8), so that it fetches whole cache lines and the operand reads
+//     (row m0 + 16 mb + l % 16, columns 16 (l / 16) + 8 h .. + 7 for half h) are free of
+//     bank conflicts;
 //   * weight fragment (strip sb): the strip layout's 1 KiB block, lane l carries
 //     w[n0 + 16 sb + l % 16][k + 16 (l / 16) .. + 15]  (16 int8).
-// So every MFMA operand read is one conflict-free ds_read_b128 at lane * 16.  The
+// Every MFMA operand read is one conflict-free ds_read_b128.  The
 // int8 half h of a weight fragment pairs with activation half h: together they
 // cover the stage's 64 K columns in two v_mfma_f32_16x16x32 steps.
 //
@@ -123,9 +125,9 @@ __global__ __launch_bounds__(NW * 64) void w8a16_pipe_kernel(
   for (int j = 0; j < FPW; ++j) {
     const int f = wave * FPW + j;
     if (f < XF) {
-      const int mb = f >> 1, h = f & 1;
-      const int m = min(m0 + mb * 16 + c16, M - 1);
-      src[j] = (const uint8_t*)(x + (int64_t)m * ldx + (int64_t)kc0 * 64 + 16 * g + 8 * h);
+      const int row = 8 * f + (lane >> 3);
+      const int m = min(m0 + row, M - 1);
+      src[j] = (const uint8_t*)(x + (int64_t)m * ldx + (int64_t)kc0 * 64 + 8 * swizzle8(row, lane & 7));
       stride[j] = 64 * (int64_t)sizeof(XT);
     } else {
       const int s = min(n0 / 16 + (f - XF), strips - 1);
@@ -171,11 +173,12 @@ __global__ __launch_bounds__(NW * 64) void w8a16_pipe_kernel(
       }
     }
   };
+  const int xoff = c16 * 128 + 16 * swizzle8(c16, 2 * g);  // piece 2 g of row c16; piece 2 g + 1: xoff ^ 16
   auto read = [&](V (&xa)[MB][2], i32x4_t (&wq)[NB], const uint8_t* stage) __attribute__((always_inline)) {
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
-      for (int h = 0; h < 2; ++h) xa[mb][h] = *(const V*)(stage + (2 * (wm * MB + mb) + h) * 1024 + lane * 16);
+      for (int h = 0; h < 2; ++h) xa[mb][h] = *(const V*)(stage + (wm * MB + mb) * 2048 + (h ? xoff ^ 16 : xoff));
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) wq[nb] = *(const i32x4_t*)(stage + (XF + wn * NB + nb) * 1024 + lane * 16);
   };
