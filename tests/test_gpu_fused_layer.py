@@ -236,3 +236,47 @@ def test_fused_errors(ops):
         x.data_ptr(), _lib.BF16, 2, k, k, 7, None, 0.0, qs.data_ptr(), n, s.data_ptr(), _lib.BF16, None,
         None, 0, buf.data_ptr(), n, 0, None, 0, None)
     assert st != 0 and "prologue" in _lib.last_error()
+
+
+# (m, n, k): tiles of 32 x 64 with one and two chunks a stage, whole and split K, ragged rows and
+# columns; then each 8-wave tile of the automatic choice.
+TILE_EPILOGUES = [(65, 100, 192), (17, 4128, 64), (70, 2048, 6144), (129, 1056, 1024), (1003, 2048, 128),
+                  (1003, 4096, 64), (1000, 6400, 64), (1003, 12288, 64)]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("m,n,k", TILE_EPILOGUES)
+def test_tile_residual_epilogue(ops, m, n, k, dtype):
+    """Past the decode rows the residual rides in the tile kernel's epilogue: bit for bit torch's
+    ``residual + linear(x)`` on the plain GEMM, in place and with a row stride of its own."""
+    q, s, qs = _weights(ops, n, k, dtype, 3)
+    g = torch.Generator(device="cuda").manual_seed(m)
+    x = torch.randn(m, k, device="cuda", generator=g).to(dtype)
+    b = torch.randn(n, device="cuda", generator=g).to(dtype)
+    for pad in (0, 3):  # 3: rows that are not 8-byte aligned
+        res = torch.randn(m, n + pad, device="cuda", generator=g).to(dtype)[:, :n]
+        for bias in (None, b):
+            want = res + ops.w8a16_gemm_strips(x, qs, n, s, bias)
+            assert torch.equal(ops.w8a16_fused_gemm_strips(x, qs, n, s, bias, residual=res), want)
+    same = res.clone()
+    ops.w8a16_fused_gemm_strips(x, qs, n, s, b, residual=same, out=same)
+    assert torch.equal(same, want)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("m,n,k", [(m, n // 32 * 32, k) for m, n, k in TILE_EPILOGUES])
+def test_tile_silu_pair_epilogue(ops, m, n, k, dtype):
+    """GatedMLP's activation in the tile kernel's epilogue: bit for bit silu_mul of the plain tile
+    GEMM, after a plain input or a separate RMSNorm."""
+    from qtts_amd import _lib
+    q, s, qs = _weights(ops, n, k, dtype, 4)
+    g = torch.Generator(device="cuda").manual_seed(m)
+    x = torch.randn(m, k, device="cuda", generator=g).to(dtype)
+    nw = (1 + 0.1 * torch.randn(k, device="cuda", generator=g)).to(dtype)
+    for bias in (None, torch.randn(n, device="cuda", generator=g).to(dtype)):
+        for norm in (False, True):
+            h = ops.rms_norm(x, nw) if norm else x
+            # the automatic tile at every row count (the plain automatic choice keeps small weights on the skinny kernel)
+            want = ops.silu_mul(ops.w8a16_gemm_strips(h, qs, n, s, bias, _lib.algo_code(_lib.ALGO_TILE)))
+            kw = {"prologue": ops.PRO_RMS_NORM, "norm_weight": nw} if norm else {}
+            assert torch.equal(ops.w8a16_gate_up_silu_strips(x, qs, n, s, bias, **kw), want)

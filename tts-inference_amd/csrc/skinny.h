@@ -580,6 +580,11 @@ struct SkinnyCfg { int mb, waves, cpw, S, cps, strips; };
 constexpr int kSkinnyMaxM = 64, kSkinnyAutoMaxM = 32;
 constexpr int64_t kSkinnyAutoMaxBytes = 9 << 20, kSkinnyAutoMaxK = 2048;
 
+// Whether the automatic choice keeps 17-32 rows on the skinny kernel's two m-blocks.
+inline bool skinny_auto_wide(int64_t m, int64_t n, int64_t k) {
+  return m > 16 && m <= kSkinnyAutoMaxM && n * k <= kSkinnyAutoMaxBytes && k <= kSkinnyAutoMaxK;
+}
+
 // m-blocks of 16 activation rows a skinny call carries.
 inline int skinny_mb(int64_t m) { return m <= 16 ? 1 : (m <= 32 ? 2 : 4); }
 

@@ -66,13 +66,21 @@ __device__ __forceinline__ float scale_bits_to_f32(uint32_t b, int dt) {
 
 template <typename XT> __device__ __forceinline__ float xbits_to_f32(uint32_t b) { return to_f32(XT{(uint16_t)b}); }
 
+// Epilogues: kEpiRes: y = residual + the output rounded to XT first (`residual + linear(x)`; y may be
+// the residual); kEpiPair: GatedMLP's activation of a fused gate_up weight (gate rows, then up rows):
+// each 16-column strip of a tile holds eight gate rows and the matching up rows, as the decode
+// kernel's half-strip pair does (skinny.h: PAIR), and y is [M, N / 2].
+enum : int { kEpiNone = 0, kEpiRes = 1, kEpiPair = 2 };
+
 // CPS: chunks a stage (2: half the stage barriers and load waits of a small-K call; the host
 // keeps every split's chunk count a multiple of it).
-template <typename XT, int BM, int BN, int P, int WM, bool F8W, bool PF = false, int NW = 4, int CPS = 1>
+template <typename XT, int BM, int BN, int P, int WM, bool F8W, bool PF = false, int NW = 4, int CPS = 1,
+          int EPI = kEpiNone>
 __global__ __launch_bounds__(NW * 64) void w8a16_pipe_kernel(
     const XT* __restrict__ x, int M, int K, int64_t ldx, const int8_t* __restrict__ qs, int N,
-    const void* __restrict__ scale, int sdt, const XT* __restrict__ bias, XT* __restrict__ y, int64_t ldy,
-    float* __restrict__ part, unsigned* __restrict__ counters, int mtiles, int ntiles, int S, int cps) {
+    const void* __restrict__ scale, int sdt, const XT* __restrict__ bias, XT* y, int64_t ldy,
+    float* __restrict__ part, unsigned* __restrict__ counters, int mtiles, int ntiles, int S, int cps, const XT* res,
+    int64_t ldr) {
   typedef mfma16<XT> MM;
   typedef typename MM::vec V;
   constexpr int WN = NW / WM;          // the NW waves form a WM x WN grid over the tile
@@ -113,10 +121,37 @@ __global__ __launch_bounds__(NW * 64) void w8a16_pipe_kernel(
   // they would cost 8 NB registers a lane, enough to cut the larger tiles' occupancy.
   uint32_t my_sc = 0u, my_bi = 0u;
   if (tid < BN) {
-    const int n = min(n0 + tid, N - 1);
+    int n = min(n0 + tid, N - 1);
+    if constexpr (EPI == kEpiPair) {  // column i of strip s: gate row 8 s + i, or the up row of i - 8
+      const int s = min((n0 + tid) >> 4, strips - 1), i = tid & 15;
+      n = 8 * s + (i & 7) + (i < 8 ? 0 : N >> 1);
+    }
     my_sc = load_scale_bits(scale, sdt, n);
     my_bi = __hip_atomic_load((uint16_t*)(bias ? bias : y) + n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
   }
+  // The residual's bits, four columns a block: before the K loop where they cost at most 16 registers
+  // a lane, else in the epilogue, all of them before the first is needed.
+  constexpr bool kResEarly = EPI == kEpiRes && NB * MB <= 8;
+  uint64_t rb[EPI == kEpiRes ? NB : 1][EPI == kEpiRes ? MB : 1];
+  auto load_res = [&]() __attribute__((always_inline)) {
+    const bool vec = ((uintptr_t)res & 7) == 0 && ldr % 4 == 0 && N % 4 == 0;  // uniform
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb) {
+        const XT* row = res + (int64_t)min(m0 + (wm * MB + mb) * 16 + c16, M - 1) * ldr;
+        const int n = n0 + (wn * NB + nb) * 16 + 4 * g;
+        if (vec) {
+          rb[nb][mb] = __hip_atomic_load((uint64_t*)(row + min(n, N - 4)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        } else {
+          uint64_t b = 0;
+#pragma unroll
+          for (int t = 0; t < 4; ++t) b |= (uint64_t)row[min(n + t, N - 1)].bits << (16 * t);
+          rb[nb][mb] = b;
+        }
+      }
+  };
+  if constexpr (kResEarly) load_res();
 
   // This wave's fragments: per-lane source at chunk kc0 and the per-chunk stride.
   const uint8_t* src[FPW];
@@ -131,7 +166,12 @@ __global__ __launch_bounds__(NW * 64) void w8a16_pipe_kernel(
       stride[j] = 64 * (int64_t)sizeof(XT);
     } else {
       const int s = min(n0 / 16 + (f - XF), strips - 1);
-      src[j] = (const uint8_t*)qs + ((int64_t)s * nchunks + kc0) * 1024 + lane * 16;
+      if constexpr (EPI == kEpiPair) {  // (N % 32 == 0: both halves sit in whole strips)
+        const int R = 8 * s + (c16 & 7) + (c16 < 8 ? 0 : N >> 1);
+        src[j] = (const uint8_t*)qs + ((int64_t)(R >> 4) * nchunks + kc0) * 1024 + ((R & 15) + 16 * g) * 16;
+      } else {
+        src[j] = (const uint8_t*)qs + ((int64_t)s * nchunks + kc0) * 1024 + lane * 16;
+      }
       stride[j] = 1024;
     }
   }
@@ -280,8 +320,13 @@ __global__ __launch_bounds__(NW * 64) void w8a16_pipe_kernel(
         for (int t = 0; t < 4; ++t) acc[nb][mb][t] = a[(nb * MB + mb) * 4 + t];
   }
 
+  if constexpr (EPI == kEpiRes && !kResEarly) load_res();
+
   // D of each 16x16 MFMA: lane (c16, g) holds rows 4g..4g+3 (weight rows n) of
   // column c16 (activation row m): four consecutive outputs of one row of y.
+  // kEpiPair: lanes g < 2 hold gate rows 4g..4g+3 of a strip and lanes g + 2 the matching up rows.
+  // One swap of the half waves per two values leaves rows 4g, 4g+1 of both with the lower lanes and
+  // rows 4g+2, 4g+3 with the upper ones, so that every lane computes two activations.
 #pragma unroll
   for (int nb = 0; nb < NB; ++nb) {
     const int nbase = n0 + (wn * NB + nb) * 16 + 4 * g;
@@ -300,6 +345,29 @@ __global__ __launch_bounds__(NW * 64) void w8a16_pipe_kernel(
       float v[4];
 #pragma unroll
       for (int t = 0; t < 4; ++t) v[t] = bias ? acc[nb][mb][t] * sc[t] + bi[t] : acc[nb][mb][t] * sc[t];
+      if constexpr (EPI == kEpiPair) {
+        const int s = (n0 >> 4) + wn * NB + nb;
+        uint16_t o[2];
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+          const auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(round_through<XT>(v[t])),
+                                                          __float_as_uint(round_through<XT>(v[t + 2])), false, false);
+          o[t] = from_f32<XT>(silu_mul<XT>(__uint_as_float(p[0]), __uint_as_float(p[1]))).bits;
+        }
+        if (s >= strips) continue;
+        XT* yo = yr + 8 * s + 4 * (g & 1) + (g & 2);
+        if (((uintptr_t)yo & 3) == 0) {
+          *(uint32_t*)yo = o[0] | ((uint32_t)o[1] << 16);
+        } else {
+          yo[0] = XT{o[0]};
+          yo[1] = XT{o[1]};
+        }
+        continue;
+      }
+      if constexpr (EPI == kEpiRes) {
+#pragma unroll
+        for (int t = 0; t < 4; ++t) v[t] = xbits_to_f32<XT>((uint32_t)(rb[nb][mb] >> (16 * t)) & 0xffffu) + round_through<XT>(v[t]);
+      }
       const uint32_t lo = pack2_f32<XT>(v[0], v[1]), hi = pack2_f32<XT>(v[2], v[3]);
       if (nbase + 3 < N && ((uintptr_t)(yr + nbase) & 7) == 0) {
         *(uint2*)(yr + nbase) = make_uint2(lo, hi);
@@ -456,18 +524,18 @@ inline void launch_pipe_p(const PipeCfg& c, const PipeArgs& a, unsigned blocks, 
       if (c.cps2) {
         qtts::launch(&w8a16_pipe_kernel<XT, BM, BN, P, WM, F8W, true, 4, 2>, dim3(blocks), dim3(256), 0, st,
                      (const XT*)a.x, (int)a.m, (int)a.k, a.ldx, a.qs, (int)a.n, a.scale, a.sdt, (const XT*)a.bias,
-                     (XT*)a.y, a.ldy, a.part, a.counters, c.mtiles, c.ntiles, c.S, c.cps);
+                     (XT*)a.y, a.ldy, a.part, a.counters, c.mtiles, c.ntiles, c.S, c.cps, (const XT*)nullptr, (int64_t)0);
         return;
       }
     }
     if (c.pf)
       qtts::launch(&w8a16_pipe_kernel<XT, BM, BN, P, WM, F8W, true>, dim3(blocks), dim3(256), 0, st, (const XT*)a.x,
                    (int)a.m, (int)a.k, a.ldx, a.qs, (int)a.n, a.scale, a.sdt, (const XT*)a.bias, (XT*)a.y, a.ldy, a.part,
-                   a.counters, c.mtiles, c.ntiles, c.S, c.cps);
+                   a.counters, c.mtiles, c.ntiles, c.S, c.cps, (const XT*)nullptr, (int64_t)0);
     else
       qtts::launch(&w8a16_pipe_kernel<XT, BM, BN, P, WM, F8W>, dim3(blocks), dim3(256), 0, st, (const XT*)a.x, (int)a.m,
                    (int)a.k, a.ldx, a.qs, (int)a.n, a.scale, a.sdt, (const XT*)a.bias, (XT*)a.y, a.ldy, a.part,
-                   a.counters, c.mtiles, c.ntiles, c.S, c.cps);
+                   a.counters, c.mtiles, c.ntiles, c.S, c.cps, (const XT*)nullptr, (int64_t)0);
   }
 }
 
@@ -502,7 +570,7 @@ inline void launch_pipe8_p(const PipeCfg& c, const PipeArgs& a, unsigned blocks,
     if constexpr (P * pipe_stage_bytes_c(BM, BN) + 64 <= kLdsBytes)                                                \
       qtts::launch(&w8a16_pipe_kernel<XT, BM, BN, P, WM, F8W, PF, 8>, dim3(blocks), dim3(512), 0, st,              \
                    (const XT*)a.x, (int)a.m, (int)a.k, a.ldx, a.qs, (int)a.n, a.scale, a.sdt, (const XT*)a.bias,   \
-                   (XT*)a.y, a.ldy, a.part, a.counters, c.mtiles, c.ntiles, c.S, c.cps);                           \
+                   (XT*)a.y, a.ldy, a.part, a.counters, c.mtiles, c.ntiles, c.S, c.cps, (const XT*)nullptr, (int64_t)0); \
   } while (0)
   if constexpr (BN == 384) {  // built with 3 stages and no read-ahead only (the launcher checks)
     QTTS_P8(3, false);

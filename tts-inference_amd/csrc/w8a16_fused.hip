@@ -16,8 +16,9 @@
 //    GEMM writes t into the workspace: y may be the residual itself).
 //  * qtts_launch_w8a16_fused: one skinny launch with the prologue computed while the
 //    activation row is staged in LDS and the residual added in the epilogue
-//    (skinny.h: PRO, RES) when the call allows it, otherwise the separate kernels
-//    around the plain W8A16 GEMM.  Fused: SiLU for one row (for two rows it no longer
+//    (skinny.h: PRO, RES) when the call allows it; past the decode rows the separate
+//    prologue and one tile launch with the residual in its epilogue (tile_fused.hip);
+//    otherwise the separate kernels around the plain W8A16 GEMM.  Fused: SiLU for one row (for two rows it no longer
 //    hides under the weight stream: talker down 9.4 us fused against 9.0 us for the
 //    two passes at M = 2; 7.0 against 9.1 us at M = 1); RMSNorm for up to 16 rows without
 //    a split-K (every workgroup needs the whole row's sum); the residual for up to 16
@@ -164,6 +165,9 @@ int qtts_launch_w8a16(const void* x, int x_dtype, int64_t m, int64_t k, int64_t 
                       int64_t ldy, int algo, void* ws, int64_t ws_bytes, hipStream_t st);
 int64_t qtts_w8a16_ws_bytes(int64_t m, int64_t n, int64_t k, int algo);
 int qtts_w8a16_xrows_built(int waves, int cpw);
+int qtts_launch_w8a16_pipe_epi(const void* x, int x_dtype, int64_t m, int64_t k, int64_t ldx, const int8_t* qs,
+                               int64_t n, const void* scale, int sdt, const void* bias, const void* res, int64_t ldr,
+                               void* y, int64_t ldy, void* ws, int64_t ws_bytes, hipStream_t st);
 
 int qtts_launch_silu_mul(const void* gu, int x_dtype, int64_t m, int64_t k, int64_t ld, void* h, int64_t ldh,
                          hipStream_t st) {
@@ -446,6 +450,14 @@ int qtts_launch_w8a16_fused(const void* x, int x_dtype, int64_t m, int64_t k, in
   if (!ws || avail < t_bytes)
     return qtts_set_error(QTTS_ERR_WORKSPACE, "w8a16 fused: workspace of %lld bytes < %lld needed",
                           (long long)ws_bytes, (long long)qtts_w8a16_fused_ws_bytes(m, n, k, algo, x_dtype));
+  // Past the decode rows: the residual in the tile kernel's epilogue, where the plain GEMM takes that
+  // kernel (w8a16.hip launch_fast), so that a fused call and the plain GEMM give the same bits.
+  if (kernel_ok && algo == QTTS_ALGO_AUTO && m > 16 && skinny_row_parts_sub(m, n, k) == 1 &&
+      !skinny_auto_wide(m, n, k) && (uintptr_t)xin % 16 == 0 && ldin % 8 == 0) {
+    const int rc = qtts_launch_w8a16_pipe_epi(xin, x_dtype, m, k, ldin, qs, n, scale, sdt, bias, res, ldr, y, ldy, ws,
+                                              avail, st);
+    if (rc != 1) return rc;
+  }
   avail = (avail - t_bytes) & ~(int64_t)255;
   void* t = (char*)ws + avail;
   const int rc = qtts_launch_w8a16(xin, x_dtype, m, k, ldin, qs, n, 0, kLayoutStrips, scale, sdt, bias, t, n, algo, ws,
@@ -469,8 +481,9 @@ int64_t qtts_w8a16_silu_ws_bytes(int64_t m, int64_t n, int64_t k, int algo, int 
 // (qtts/layers/activation.py:142-147): x [m, k]; prologue none or RMSNorm (nw, eps);
 // qs the fused [n, k] gate_up weight (gate rows then up rows, n % 2 == 0); act [m, n/2]
 // with row stride ldact.  Up to 16 decode rows (n % 32 == 0): one launch, the activation
-// in the GEMM's epilogue.  Otherwise the norm, the GEMM into the workspace and
-// silu_mul run one after another.
+// in the GEMM's epilogue.  Past them (automatic choice, n % 32 == 0) the norm, then one tile
+// launch with the activation in its epilogue (tile_fused.hip).  Otherwise the norm, the GEMM
+// into the workspace and silu_mul run one after another.
 int qtts_launch_w8a16_gate_up_silu(const void* x, int x_dtype, int64_t m, int64_t k, int64_t ldx, int pro,
                                    const void* nw, float eps, const int8_t* qs, int64_t n, const void* scale, int sdt,
                                    const void* bias, void* act, int64_t ldact, int algo, void* ws, int64_t ws_bytes,
@@ -506,6 +519,25 @@ int qtts_launch_w8a16_gate_up_silu(const void* x, int x_dtype, int64_t m, int64_
                           (long long)ws_bytes, (long long)qtts_w8a16_fused_ws_bytes(m, n, k, algo, x_dtype));
   const int64_t avail = (ws_bytes - g_bytes) & ~(int64_t)255;
   void* gu = (char*)ws + avail;
+  // Past the decode rows: the norm, then one tile launch with the activation in its epilogue.
+  if (kernel_ok && x_aligned && algo == QTTS_ALGO_AUTO && m > 16 && n % 32 == 0) {
+    const void* xin = x;
+    int64_t ldin = ldx, left = avail;
+    if (pro == kProRmsNorm) {
+      const int64_t h_bytes = al256(m * k * esize(x_dtype));
+      if (avail < kCounterBytes + h_bytes)
+        return qtts_set_error(QTTS_ERR_WORKSPACE, "w8a16 fused: workspace of %lld bytes < %lld needed",
+                              (long long)avail, (long long)qtts_w8a16_fused_ws_bytes(m, n, k, algo, x_dtype));
+      left = (avail - h_bytes) & ~(int64_t)255;
+      xin = (char*)ws + left;
+      ldin = k;
+      const int nrc = qtts_launch_rms_norm(x, x_dtype, m, k, ldx, nw, eps, (void*)xin, k, st);
+      if (nrc != QTTS_OK) return nrc;
+    }
+    const int rc = qtts_launch_w8a16_pipe_epi(xin, x_dtype, m, k, ldin, qs, n, scale, sdt, bias, nullptr, 0, act, ldact,
+                                              ws, left, st);
+    if (rc != 1) return rc;
+  }
   int rc = qtts_launch_w8a16_fused(x, x_dtype, m, k, ldx, pro, nw, eps, qs, n, scale, sdt, bias, nullptr, 0, gu, n,
                                    algo, ws, avail, st);
   if (rc != QTTS_OK) return rc;
