@@ -280,3 +280,69 @@ def test_tile_silu_pair_epilogue(ops, m, n, k, dtype):
             want = ops.silu_mul(ops.w8a16_gemm_strips(h, qs, n, s, bias, _lib.algo_code(_lib.ALGO_TILE)))
             kw = {"prologue": ops.PRO_RMS_NORM, "norm_weight": nw} if norm else {}
             assert torch.equal(ops.w8a16_gate_up_silu_strips(x, qs, n, s, bias, **kw), want)
+
+
+# (m, n, k): row edges of the 16-row blocks (with 5 rows for the norm inside), ragged columns, each built K
+WIDE = [(5, 4096, 1024), (9, 4096, 1024), (16, 100, 1024), (17, 6144, 1024), (33, 4096, 1024), (48, 1040, 1024),
+        (65, 6144, 1024), (96, 6144, 1024), (128, 6144, 1024), (9, 12288, 2048), (31, 12288, 2048), (47, 4096, 2048),
+        (128, 4096, 2048), (27, 2048, 2048), (127, 2048, 2048), (12, 1000, 3072), (97, 1024, 3072), (13, 2048, 6144),
+        (32, 2048, 6144), (64, 2048, 6144)]
+
+
+def _ref64(h, q, s, b):
+    """The dequantize-then-matmul of the packed codes in float64 (torch on the GPU: the oracle's formula, faster)."""
+    y = h.double() @ (q.double() * s.double()[:, None]).t()
+    return (y if b is None else y + b.double()).cpu().numpy()
+
+
+def _bar_product(y, gate, up, what):
+    """The GEMM bar carried through silu(g) * u to first order: |d silu| <= 1.1 |dg|, half an output ulp each for the
+    roundings of g, u and silu(g) in between."""
+    def half(v):
+        return 2.0 ** (np.floor(np.log2(np.maximum(np.abs(v), 1e-30))) - 7) / 2
+    rms_g, rms_u = (np.sqrt(np.mean(v * v)) for v in (gate, up))
+    silu = gate / (1 + np.exp(-gate))
+    dg, du = 1e-2 * rms_g + half(gate), 1e-2 * rms_u + half(up)
+    bound = (1.1 * dg + half(silu)) * np.abs(up) + np.abs(silu) * du + 1.1 * dg * du + half(silu * up)
+    err = np.abs(y - silu * up)
+    assert (err <= bound).all(), f"{what}: {err.max()} {int((err > bound).sum())}"
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("m,n,k", WIDE)
+def test_wide_calls(ops, m, n, k, dtype):
+    """The automatic choice at 9-128 rows (the one-round tiles): every form against float64, the
+    residual bit for bit the plain call's, strided rows, and rows that do not meet (a row of infinities and
+    one of NaN leave the others' bits alone)."""
+    q, s, qs = _weights(ops, n, k, dtype, 5)
+    g = torch.Generator(device="cuda").manual_seed(m * 7 + k)
+    x = torch.randn(m, k + 8, device="cuda", generator=g).to(dtype)[:, :k]
+    b = torch.randn(n, device="cuda", generator=g).to(dtype)
+    nw = (1 + 0.1 * torch.randn(k, device="cuda", generator=g)).to(dtype)
+    what = f"wide m={m} n={n} k={k} {dtype}"
+    y = ops.w8a16_gemm_strips(x, qs, n, s, b)
+    assert_close(y, _ref64(x, q, s, b), what)
+    res = torch.randn(m, n + 3, device="cuda", generator=g).to(dtype)[:, :n]
+    assert torch.equal(ops.w8a16_fused_gemm_strips(x, qs, n, s, b, residual=res), res + y), what
+    hn = _round(O.rms_norm(_bits(x.contiguous()), _bits(nw), 1e-6, _TD[dtype]), dtype).cuda()
+    yn = ops.w8a16_fused_gemm_strips(x, qs, n, s, None, prologue=ops.PRO_RMS_NORM, norm_weight=nw)
+    assert_close(yn, _ref64(hn, q, s, None), what + " norm")
+    odd = x.clone()
+    odd[0], odd[m // 2] = float("inf"), float("nan")
+    rest = [i for i in range(m) if i not in (0, m // 2)]
+    assert torch.equal(ops.w8a16_gemm_strips(odd, qs, n, s, b)[rest], y[rest]), what
+    if n % 32 == 0:
+        for h, kw in ((x, {}), (hn, {"prologue": ops.PRO_RMS_NORM, "norm_weight": nw})):
+            full = _ref64(h, q, s, b)
+            act = ops.w8a16_gate_up_silu_strips(x, qs, n, s, b, **kw)
+            _bar_product(act.double().cpu().numpy(), full[:, : n // 2], full[:, n // 2:], what + str(list(kw)))
+
+
+@pytest.mark.parametrize("m,n,k", [(9, 4096, 1024), (33, 6144, 1024), (47, 4096, 2048), (97, 1024, 3072), (64, 2048, 6144)])
+def test_wide_fp8_codes(ops, m, n, k):
+    """The same kernel on e4m3 codes: against float64."""
+    g = torch.Generator(device="cuda").manual_seed(m + n)
+    w = (torch.randn(n, k, device="cuda", generator=g) * 0.02).to(torch.bfloat16)
+    q, s = ops.pack_fp8(w)
+    x = torch.randn(m, k, device="cuda", generator=g).to(torch.bfloat16)
+    assert_close(ops.fp8w_gemm_strips(x, ops.fp8w_strips(q), n, s), _ref64(x, q.float(), s, None), f"wide fp8 {m} {n} {k}")

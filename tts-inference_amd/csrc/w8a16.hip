@@ -14,6 +14,7 @@
 //    epilogue's scale and bias are fetched first, so a call costs one memory round
 //    trip.  Waves meet in LDS; workgroups that split K further meet through the
 //    workspace (splitk.h) with no second launch.
+//  * wide (9-128 rows where one round of workgroups covers the call): wide.h.
 //  * tile (M > 16, prefill rows): LDS-tiled bf16 MFMA GEMM, BM x 128 x 64 tiles,
 //    4 waves in 2x2, double-buffered LDS; the weight tile is dequantized to bf16 on
 //    its way into LDS.
@@ -273,6 +274,10 @@ int qtts_launch_w8a16_skinny_sub(const void* x, int x_dtype, int64_t m, int64_t 
                                  int64_t n, const void* scale, int sdt, const void* bias, void* y, int64_t ldy,
                                  int sub, int waves, int cpw, unsigned blocks, hipStream_t st);
 
+int qtts_launch_w8a16_wide(const void* x, int x_dtype, int64_t m, int64_t k, int64_t ldx, const int8_t* qs, int64_t n,
+                           const void* scale, int sdt, const void* bias, const void* res, int64_t ldr, void* y,
+                           int64_t ldy, hipStream_t st);
+
 int64_t qtts_w8a16_ws_bytes(int64_t m, int64_t n, int64_t k, int algo) {
   const int family = algo & 0xff, splits = (algo >> 8) & 0xff, waves = (algo >> 16) & 0xff;
   int64_t ws = 0;
@@ -294,6 +299,12 @@ static int launch_fast(const XT* x, int64_t m, int64_t k, int64_t ldx, const int
   int family = algo & 0xff;
   const int splits = (algo >> 8) & 0xff, waves = (algo >> 16) & 0xff;
   const bool wide_ok = LAYOUT == kLayoutStrips && k % 64 == 0;  // skinny beyond 16 rows
+  // 9 to 128 rows that one round of the wide kernel's workgroups covers (wide_rule.h)
+  if (LAYOUT == kLayoutStrips && algo == QTTS_ALGO_AUTO) {
+    const int rc = qtts_launch_w8a16_wide(x, std::is_same<XT, bf16_t>::value ? QTTS_BF16 : QTTS_F16, m, k, ldx, q, n,
+                                          scale, sdt, bias, nullptr, 0, y, ldy, st);
+    if (rc != 1) return rc;
+  }
   // Row-split strips: requested by family, or the automatic choice for staged decode rows
   // where the strips alone would leave compute units idle.
   int sub = family == QTTS_ALGO_SKINNY_HALF ? 2 : (family == QTTS_ALGO_SKINNY_QUARTER ? 4 : 1);

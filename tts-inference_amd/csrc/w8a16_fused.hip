@@ -26,6 +26,7 @@
 //    sum in different orders: the fused
 //    result is within the GEMM tolerance of the separate one, not bit-identical.
 #include "skinny_fused.h"
+#include "wide_rule.h"
 
 using namespace qtts;
 
@@ -168,6 +169,13 @@ int qtts_w8a16_xrows_built(int waves, int cpw);
 int qtts_launch_w8a16_pipe_epi(const void* x, int x_dtype, int64_t m, int64_t k, int64_t ldx, const int8_t* qs,
                                int64_t n, const void* scale, int sdt, const void* bias, const void* res, int64_t ldr,
                                void* y, int64_t ldy, void* ws, int64_t ws_bytes, hipStream_t st);
+
+int qtts_launch_w8a16_wide(const void* x, int x_dtype, int64_t m, int64_t k, int64_t ldx, const int8_t* qs, int64_t n,
+                           const void* scale, int sdt, const void* bias, const void* res, int64_t ldr, void* y,
+                           int64_t ldy, hipStream_t st);
+int qtts_launch_w8a16_wide_fused(const void* x, int x_dtype, int64_t m, int64_t k, int64_t ldx, const void* nw, float eps,
+                                 const int8_t* qs, int64_t n, const void* scale, int sdt, const void* bias, bool pair,
+                                 void* y, int64_t ldy, hipStream_t st);
 
 int qtts_launch_silu_mul(const void* gu, int x_dtype, int64_t m, int64_t k, int64_t ld, void* h, int64_t ldh,
                          hipStream_t st) {
@@ -413,6 +421,10 @@ int qtts_launch_w8a16_fused(const void* x, int x_dtype, int64_t m, int64_t k, in
   // 1. The prologue inside the GEMM: SiLU * mul for one row, RMSNorm for up to 16.
   if (pro != kProNone && kernel_ok && x_aligned &&
       ((pro == kProSiluMul && m == 1) || (pro == kProRmsNorm && m <= 16 && !res && (uintptr_t)nw % 16 == 0))) {
+    if (pro == kProRmsNorm && algo == QTTS_ALGO_AUTO) {
+      const int rc = qtts_launch_w8a16_wide_fused(x, x_dtype, m, k, ldx, nw, eps, qs, n, scale, sdt, bias, false, y, ldy, st);
+      if (rc != 1) return rc;
+    }
     a.x = x;
     a.ldx = ldx;
     const int rc = try_fused(pro, res != nullptr, a, x_dtype, sdt, algo, ws, ws_bytes);
@@ -426,6 +438,11 @@ int qtts_launch_w8a16_fused(const void* x, int x_dtype, int64_t m, int64_t k, in
     if (!ws || ws_bytes < kCounterBytes + h_bytes)
       return qtts_set_error(QTTS_ERR_WORKSPACE, "w8a16 fused: workspace of %lld bytes < %lld needed",
                             (long long)ws_bytes, (long long)qtts_w8a16_fused_ws_bytes(m, n, k, algo, x_dtype));
+    if (pro == kProRmsNorm && kernel_ok && x_aligned && algo == QTTS_ALGO_AUTO && m > 16 && !res && (uintptr_t)nw % 16 == 0) {
+      // past the decode rows, the norm inside the wide kernel
+      const int rc = qtts_launch_w8a16_wide_fused(x, x_dtype, m, k, ldx, nw, eps, qs, n, scale, sdt, bias, false, y, ldy, st);
+      if (rc != 1) return rc;
+    }
     avail = (ws_bytes - h_bytes) & ~(int64_t)255;
     void* h = (char*)ws + avail;
     const int rc = pro == kProSiluMul ? qtts_launch_silu_mul(x, x_dtype, m, k, ldx, h, k, st)
@@ -435,7 +452,12 @@ int qtts_launch_w8a16_fused(const void* x, int x_dtype, int64_t m, int64_t k, in
     ldin = k;
   }
   // 3. The residual in the GEMM's epilogue (up to 16 staged rows, up to 64 on half strips).
-  if (res && kernel_ok && m <= kRowPartsMaxM && (uintptr_t)xin % 16 == 0 && (m == 1 || ldin % 8 == 0)) {
+  const bool wide = kernel_ok && algo == QTTS_ALGO_AUTO && wide_cfg(m, n, k).mb > 0 && (uintptr_t)xin % 16 == 0 && ldin % 8 == 0;
+  if (res && wide && m <= 16) {
+    const int rc = qtts_launch_w8a16_wide(xin, x_dtype, m, k, ldin, qs, n, scale, sdt, bias, res, ldr, y, ldy, st);
+    if (rc != 1) return rc;
+  }
+  if (res && kernel_ok && !wide && m <= kRowPartsMaxM && (uintptr_t)xin % 16 == 0 && (m == 1 || ldin % 8 == 0)) {
     a.x = xin;
     a.ldx = ldin;
     const int rc = try_fused(kProNone, true, a, x_dtype, sdt, algo, ws, avail);
@@ -450,6 +472,10 @@ int qtts_launch_w8a16_fused(const void* x, int x_dtype, int64_t m, int64_t k, in
   if (!ws || avail < t_bytes)
     return qtts_set_error(QTTS_ERR_WORKSPACE, "w8a16 fused: workspace of %lld bytes < %lld needed",
                           (long long)ws_bytes, (long long)qtts_w8a16_fused_ws_bytes(m, n, k, algo, x_dtype));
+  if (wide) {
+    const int rc = qtts_launch_w8a16_wide(xin, x_dtype, m, k, ldin, qs, n, scale, sdt, bias, res, ldr, y, ldy, st);
+    if (rc != 1) return rc;
+  }
   // Past the decode rows: the residual in the tile kernel's epilogue, where the plain GEMM takes that
   // kernel (w8a16.hip launch_fast), so that a fused call and the plain GEMM give the same bits.
   if (kernel_ok && algo == QTTS_ALGO_AUTO && m > 16 && skinny_row_parts_sub(m, n, k) == 1 &&
@@ -493,6 +519,12 @@ int qtts_launch_w8a16_gate_up_silu(const void* x, int x_dtype, int64_t m, int64_
   const bool kernel_ok = k % 64 == 0 && x_dtype != QTTS_F32 && (sdt == x_dtype || sdt == QTTS_F32) &&
                          family != QTTS_ALGO_TILE && !direct_x;
   const bool x_aligned = (uintptr_t)x % 16 == 0 && (m == 1 || ldx % 8 == 0);
+  const bool wide_pair = kernel_ok && x_aligned && algo == QTTS_ALGO_AUTO && n % 32 == 0 && ldx % 8 == 0;
+  if (wide_pair && m <= 16 && (pro == kProNone || (uintptr_t)nw % 16 == 0)) {
+    const int rc = qtts_launch_w8a16_wide_fused(x, x_dtype, m, k, ldx, pro == kProNone ? nullptr : nw, eps, qs, n, scale, sdt,
+                                                bias, true, act, ldact, st);
+    if (rc != 1) return rc;
+  }
   if (kernel_ok && x_aligned && (pro == kProNone || (uintptr_t)nw % 16 == 0)) {
     FusedArgs a{};
     a.x = x;
@@ -519,8 +551,9 @@ int qtts_launch_w8a16_gate_up_silu(const void* x, int x_dtype, int64_t m, int64_
                           (long long)ws_bytes, (long long)qtts_w8a16_fused_ws_bytes(m, n, k, algo, x_dtype));
   const int64_t avail = (ws_bytes - g_bytes) & ~(int64_t)255;
   void* gu = (char*)ws + avail;
-  // Past the decode rows: the norm, then one tile launch with the activation in its epilogue.
-  if (kernel_ok && x_aligned && algo == QTTS_ALGO_AUTO && m > 16 && n % 32 == 0) {
+  // Past the decode rows: one wide launch with the norm and the activation, or the norm, then one wide or
+  // tile launch with the activation in its epilogue.
+  if (wide_pair && m > 16) {
     const void* xin = x;
     int64_t ldin = ldx, left = avail;
     if (pro == kProRmsNorm) {
@@ -528,14 +561,19 @@ int qtts_launch_w8a16_gate_up_silu(const void* x, int x_dtype, int64_t m, int64_
       if (avail < kCounterBytes + h_bytes)
         return qtts_set_error(QTTS_ERR_WORKSPACE, "w8a16 fused: workspace of %lld bytes < %lld needed",
                               (long long)avail, (long long)qtts_w8a16_fused_ws_bytes(m, n, k, algo, x_dtype));
+      if ((uintptr_t)nw % 16 == 0) {
+        const int rc = qtts_launch_w8a16_wide_fused(x, x_dtype, m, k, ldx, nw, eps, qs, n, scale, sdt, bias, true, act, ldact, st);
+        if (rc != 1) return rc;
+      }
       left = (avail - h_bytes) & ~(int64_t)255;
       xin = (char*)ws + left;
       ldin = k;
       const int nrc = qtts_launch_rms_norm(x, x_dtype, m, k, ldx, nw, eps, (void*)xin, k, st);
       if (nrc != QTTS_OK) return nrc;
     }
-    const int rc = qtts_launch_w8a16_pipe_epi(xin, x_dtype, m, k, ldin, qs, n, scale, sdt, bias, nullptr, 0, act, ldact,
-                                              ws, left, st);
+    int rc = qtts_launch_w8a16_wide_fused(xin, x_dtype, m, k, ldin, nullptr, eps, qs, n, scale, sdt, bias, true, act, ldact, st);
+    if (rc == 1)
+      rc = qtts_launch_w8a16_pipe_epi(xin, x_dtype, m, k, ldin, qs, n, scale, sdt, bias, nullptr, 0, act, ldact, ws, left, st);
     if (rc != 1) return rc;
   }
   int rc = qtts_launch_w8a16_fused(x, x_dtype, m, k, ldx, pro, nw, eps, qs, n, scale, sdt, bias, nullptr, 0, gu, n,

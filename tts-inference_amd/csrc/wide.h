@@ -1,0 +1,312 @@
+// The W8A16 kernel for 9 to 128 rows of weights that fill the GPU once (decode batches past 8, the code
+// predictor's prefix walk, short prompts): strip weights, K = 64 W CPW.
+//
+// These calls are bound by latency and by the bytes each compute unit pulls through L2, not by the
+// matrix cores: a ring of LDS stages (tile_w8a16.h) spends a wait and a barrier on each of its 8-48
+// stages.  Here a workgroup owns 16 MB rows x 16 NB columns and all of K; its W waves split K into
+// runs of CPW chunks, and a wave issues every load of its run before it consumes any: the activation
+// rows straight to its own LDS block in whole cache lines (16-byte pieces swizzled, as pipe.h's
+// stages), the weights to registers.  A call is one memory round trip and one reduction
+// through LDS.  (Activation operands loaded to registers in MFMA lane order, as the decode kernel's
+// direct form does, touch each line twice at half width: 0.5-1.5 us a call slower at 32 rows.)
+//
+// Measured in graphs over distinct weights (5 layers of the predictor's, 12-28 of the talker's), us a call,
+// the former automatic choice -> this kernel at 16 / 32 / 64 / 128 rows: the talker's qkv 4.83 / 6.89 /
+// 7.40 / 7.94 -> 4.01 / 4.49 / 5.52 / 6.95, o_proj 3.76 / 5.51 / 7.30 / 7.31 -> 3.64 / 3.69 / 4.30 / 5.01,
+// gate_up at 16 / 32 9.58 / 9.76 -> 7.42 / 8.30, down_proj at 32 / 64 9.48 / 9.64 -> 6.68 / 7.73; the
+// predictor's qkv 4.71 / 5.24 / 6.04 / 6.24 -> 4.32 / 4.73 / 5.13 / 6.10, o_proj 4.42 / 4.93 / 5.90 /
+// 7.94 -> 4.39 / 4.48 / 4.66 / 5.39, gate_up 5.50 / 7.18 / 6.35 / 8.11 -> 4.66 / 5.10 / 5.83 / 7.45,
+// down_proj 5.13 / 6.08 / 7.90 / 8.48 -> 4.94 / 5.03 / 5.25 / 5.94.  With the RMSNorm inside against the
+// norm before the GEMM (or the decode kernel's): predictor qkv 6.64 / 7.66 / 8.76 / 9.05 -> 5.06 / 5.50 / 6.14 /
+// 7.55, talker qkv 6.96 / 9.29 / 10.17 -> 5.88 / 6.54 / 7.88 to 64 rows; gate_up with norm and activation 8.24 /
+// 10.16 / 9.60 -> 5.72 / 6.17 / 7.48 (predictor), 13.97 -> 10.03 at 16 rows (talker).  The floor of a call
+// is the 1.6 us launch, one memory round trip and 2-13 MB at 5.1 TB/s.
+#pragma once
+
+#include <algorithm>
+#include <type_traits>
+
+#include "common.h"
+#include "layout.h"
+#include "pipe.h"
+#include "skinny.h"
+#include "tile_w8a16.h"
+#include "wide_rule.h"
+
+namespace qtts {
+
+// v + v of the lanes 16 and 32 away: the four lanes that share a row in the MFMA operand layout.
+__device__ __forceinline__ float add_row_lanes(float v) {
+  auto s = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = __uint_as_float(s[0]) + __uint_as_float(s[1]);
+  s = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return __uint_as_float(s[0]) + __uint_as_float(s[1]);
+}
+
+// EPI: tile_w8a16.h's epilogues.  NORM: the input is RMSNorm(x) with weight aux and epsilon eps,
+// rounded as the reference rounds it (skinny.h: kProRmsNorm): each wave sums x^2 over its run, the
+// waves meet at one fence-free barrier while the weights stay in flight, and each scales its operands.
+// CL: chunks of a run that go through LDS; the rest load to registers in lane order (LDS holds no more).
+// (Weights load plainly under either weight policy: the streaming form measured 0.2-0.8 us a call slower.)
+template <typename XT, int MB, int NB, int W, int CPW, int CL, int EPI, bool NORM, bool F8W>
+__global__ __launch_bounds__(W * 64) void w8a16_wide_kernel(
+    const int8_t* __restrict__ qs, const XT* __restrict__ x, const void* scale, const XT* bias, const XT* aux, int ldx,
+    int M, int N, int sdt, float eps, XT* y, int64_t ldy, const XT* res, int64_t ldr) {
+  typedef mfma16<XT> MM;
+  typedef typename MM::vec V;
+  constexpr int XI = 2 * MB * CL, P = 8 * CL;  // direct loads a wave, 16-byte pieces a row of its block
+  constexpr int nchunks = W * CPW;
+  static_assert(CL <= CPW && (CL % 2 == 0 || CL == 1 || CL == 3), "pieces in groups of 16, or of 8");
+  __shared__ __align__(1024) uint8_t lds[W][1024 * (2 * MB * CL > MB * NB ? 2 * MB * CL : MB * NB)];
+  __shared__ uint32_t epi_sc[16 * NB], epi_bi[16 * NB];  // scale and bias bits, column by column
+  __shared__ float nss[NORM ? W : 1][NORM ? 16 * MB : 1];
+  const int strips = (N + 15) >> 4;
+  const int s0 = blockIdx.x * NB, y0 = blockIdx.z * (16 * MB);
+  if (s0 >= strips) return;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r = lane & 15, g = lane >> 4;
+  const int wc0 = wave * CPW;
+
+  // Position of piece p of a row in the wave's block (an involution): conflict-free operand reads.
+  auto swz = [](int row, int p) { return CL % 2 == 0 ? p ^ (row & 15) : ((p & ~7) | swizzle8(row, p & 7)); };
+#pragma unroll
+  for (int i = 0; i < XI; ++i) {
+    const int flat = i * 64 + lane, row = flat / P, p = flat % P;
+    load_to_lds16(x + (int64_t)min(y0 + row, M - 1) * ldx + wc0 * 64 + 8 * swz(row, p), &lds[wave][i * 1024]);
+  }
+  i32x4_t w[CPW][NB], xa[CPW][MB], xb[CPW][MB], nw[NORM ? CPW : 1][2];
+#pragma unroll
+  for (int u = CL; u < CPW; ++u)
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) {
+      const XT* p = x + (int64_t)min(y0 + 16 * mb + r, M - 1) * ldx + (wc0 + u) * 64 + 16 * g;
+      xa[u][mb] = *(const i32x4_t*)p;
+      xb[u][mb] = *(const i32x4_t*)(p + 8);
+    }
+  if constexpr (NORM) {
+#pragma unroll
+    for (int u = 0; u < CPW; ++u) {
+      nw[u][0] = *(const i32x4_t*)(aux + (wc0 + u) * 64 + 16 * g);
+      nw[u][1] = *(const i32x4_t*)(aux + (wc0 + u) * 64 + 16 * g + 8);
+    }
+  }
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int nb = 0; nb < NB; ++nb) {
+    const int s = min(s0 + nb, strips - 1);
+    const int8_t* wp;
+    if constexpr (EPI == kEpiPair) {  // (N % 32 == 0: both halves sit in whole strips)
+      const int R = 8 * s + (r & 7) + (r < 8 ? 0 : (N >> 1));
+      wp = qs + ((int64_t)(R >> 4) * nchunks + wc0) * 1024 + ((R & 15) + 16 * g) * 16;
+    } else {
+      wp = qs + ((int64_t)s * nchunks + wc0) * 1024 + lane * 16;
+    }
+#pragma unroll
+    for (int u = 0; u < CPW; ++u) w[u][nb] = load_weight<false>(wp + u * 1024);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+
+  // The epilogue is shared by the waves: unit u (wave u % W) is two of the four rows a lane holds of
+  // block u / 2 (kEpiPair: a block's 16 x 8 outputs, two a lane).  Its operands are raw bits, fetched after
+  // the weights and not needed before the end; thread t < 16 NB takes column t's scale and bias
+  // (every thread loads: a branch here would end in a wait).
+  constexpr int UNITS = EPI == kEpiPair ? NB * MB : 2 * NB * MB;
+  constexpr int UPW = (UNITS + W - 1) / W;
+  uint32_t my_sc, my_bi, rb[EPI == kEpiRes ? UPW : 1][2];
+  {
+    const int t = min((int)threadIdx.x, 16 * NB - 1), s = s0 + (t >> 4), i = t & 15;
+    const int n = min(EPI == kEpiPair ? 8 * s + (i & 7) + (i < 8 ? 0 : (N >> 1)) : 16 * s + i, N - 1);
+    my_sc = load_scale_bits(scale, sdt, n);
+    my_bi = load_bits((bias ? bias : x) + (bias ? n : 0));
+    if constexpr (EPI == kEpiRes) {
+#pragma unroll
+      for (int j = 0; j < UPW; ++j) {
+        const int u = min(wave + j * W, UNITS - 1), q = u >> 1;
+        const XT* row = res + (int64_t)min(y0 + 16 * (q % MB) + r, M - 1) * ldr;
+#pragma unroll
+        for (int e = 0; e < 2; ++e)
+          rb[j][e] = load_bits(row + min(16 * (s0 + q / MB) + 4 * g + 2 * (u & 1) + e, N - 1));
+      }
+    }
+  }
+  __builtin_amdgcn_sched_barrier(0);  // every load in flight before the first wait
+
+  wait_vmcnt<CPW * NB>();  // the rows have landed; at least the weights issued after them may be in flight
+#pragma unroll
+  for (int u = 0; u < CL; ++u)
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) {
+      const int row = 16 * mb + r;
+      xa[u][mb] = *(const i32x4_t*)&lds[wave][(row * P + swz(row, 8 * u + 2 * g)) * 16];
+      xb[u][mb] = *(const i32x4_t*)&lds[wave][(row * P + swz(row, 8 * u + 2 * g + 1)) * 16];
+    }
+  if constexpr (NORM) {
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) {
+      float ss = 0.0f;
+#pragma unroll
+      for (int u = 0; u < CPW; ++u)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) ss = sq2_acc<XT>((uint32_t)xb[u][mb][i], sq2_acc<XT>((uint32_t)xa[u][mb][i], ss));
+      ss = add_row_lanes(ss);
+      if (g == 0) nss[wave][16 * mb + r] = ss;
+    }
+    wait_lgkmcnt0();
+    barrier_only();
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) {
+      float t = 0.0f;
+#pragma unroll
+      for (int v = 0; v < W; ++v) t += nss[v][16 * mb + r];
+      const float inv = 1.0f / __builtin_sqrtf(t / (float)(64 * nchunks) + eps);
+#pragma unroll
+      for (int u = 0; u < CPW; ++u)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          i32x4_t& v = h ? xb[u][mb] : xa[u][mb];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const uint32_t p = (uint32_t)v[i], q = (uint32_t)nw[u][h][i];
+            const float a = to_f32(XT{(uint16_t)p}), b = to_f32(XT{(uint16_t)(p >> 16)});
+            v[i] = (int)pack2_f32<XT>((a * inv) * to_f32(XT{(uint16_t)q}), (b * inv) * to_f32(XT{(uint16_t)(q >> 16)}));
+          }
+        }
+    }
+  }
+
+  f32x4_t acc[NB][MB];
+#pragma unroll
+  for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) acc[nb][mb] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+  for (int u = 0; u < CPW; ++u)
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) {
+      const V wlo = wcvt<F8W, XT>((uint32_t)w[u][nb][0], (uint32_t)w[u][nb][1]);
+      const V whi = wcvt<F8W, XT>((uint32_t)w[u][nb][2], (uint32_t)w[u][nb][3]);
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb) acc[nb][mb] = MM::mma(wlo, __builtin_bit_cast(V, xa[u][mb]), acc[nb][mb]);
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb) acc[nb][mb] = MM::mma(whi, __builtin_bit_cast(V, xb[u][mb]), acc[nb][mb]);
+    }
+
+  // Each wave's sums over its own rows block (its reads of it are done: the MFMAs above waited for them).
+#pragma unroll
+  for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) *(f32x4_t*)&lds[wave][((nb * MB + mb) * 64 + lane) * 16] = acc[nb][mb];
+  if ((int)threadIdx.x < 16 * NB) {
+    epi_sc[threadIdx.x] = my_sc;
+    epi_bi[threadIdx.x] = my_bi;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < UPW; ++j) {  // sums in wave order
+    const int u = wave + j * W;
+    if (u >= UNITS) break;
+    const int q = EPI == kEpiPair ? u : u >> 1;
+    const int nb = q / MB, s = s0 + nb, m = y0 + 16 * (q % MB) + r;
+    uint16_t o[2];
+    int n;
+    if constexpr (EPI == kEpiPair) {
+      // lane (r, g): columns 2 g, 2 g + 1 of the strip's 8; the gate sums sit in lane (r, g / 2), the up sums 32 lanes on
+      const int src = (q * 64 + r + 16 * (g >> 1)) * 16 + 8 * (g & 1);
+      float a[2] = {0.0f, 0.0f}, b[2] = {0.0f, 0.0f};
+#pragma unroll
+      for (int v = 0; v < W; ++v)
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          a[e] += ((const float*)&lds[v][src])[e];
+          b[e] += ((const float*)&lds[v][src + 512])[e];
+        }
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        const int cg = 16 * nb + 2 * g + e, cu = cg + 8;
+        float gv = a[e] * scale_bits_to_f32(epi_sc[cg], sdt), uv = b[e] * scale_bits_to_f32(epi_sc[cu], sdt);
+        if (bias) {
+          gv += xbits_to_f32<XT>(epi_bi[cg]);
+          uv += xbits_to_f32<XT>(epi_bi[cu]);
+        }
+        o[e] = from_f32<XT>(silu_mul<XT>(round_through<XT>(gv), round_through<XT>(uv))).bits;
+      }
+      n = 8 * s + 2 * g;
+    } else {
+      const int src = (q * 64 + lane) * 16 + 8 * (u & 1);
+      float a[2] = {0.0f, 0.0f};
+#pragma unroll
+      for (int v = 0; v < W; ++v)
+#pragma unroll
+        for (int e = 0; e < 2; ++e) a[e] += ((const float*)&lds[v][src])[e];
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        const int c = 16 * nb + 4 * g + 2 * (u & 1) + e;
+        float f = a[e] * scale_bits_to_f32(epi_sc[c], sdt);
+        if (bias) f += xbits_to_f32<XT>(epi_bi[c]);
+        if constexpr (EPI == kEpiRes) f = xbits_to_f32<XT>(rb[j][e]) + round_through<XT>(f);
+        o[e] = from_f32<XT>(f).bits;
+      }
+      n = 16 * s + 4 * g + 2 * (u & 1);
+    }
+    const int cols = EPI == kEpiPair ? N >> 1 : N;
+    if (m >= M) continue;
+    XT* yr = y + (int64_t)m * ldy + n;
+    if (n + 1 < cols && ((uintptr_t)yr & 3) == 0) {
+      *(uint32_t*)yr = o[0] | ((uint32_t)o[1] << 16);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 2; ++e)
+        if (n + e < cols) yr[e] = XT{o[e]};
+    }
+  }
+}
+
+struct WideArgs {
+  const void* x; int64_t m, ldx; const int8_t* qs; int64_t n; const void* scale; int sdt; const void* bias;
+  const void* aux; float eps; const void* res; int64_t ldr; void* y; int64_t ldy; hipStream_t st;
+};
+
+// One launch of a configuration of wide_cfg (wide_rule.h); false when it is not built.
+template <typename XT, int EPI, bool NORM, bool F8W> inline bool launch_wide(const WideCfg& c, const WideArgs& a) {
+  const int64_t strips = (a.n + 15) / 16;
+  const dim3 grid((unsigned)(((strips + c.nb - 1) / c.nb + 7) / 8 * 8), 1, (unsigned)((a.m + 16 * c.mb - 1) / (16 * c.mb)));
+#define QTTS_WIDE(MB, NB, W, CPW, CL)                                                                                \
+  if (c.mb == MB && c.nb == NB && c.waves == W && c.cpw == CPW) {                                                    \
+    qtts::launch(&w8a16_wide_kernel<XT, MB, NB, W, CPW, CL, EPI, NORM, F8W>, grid, dim3(W * 64), 0, a.st, a.qs,      \
+                 (const XT*)a.x, a.scale, (const XT*)a.bias, (const XT*)a.aux, (int)a.ldx, (int)a.m, (int)a.n, a.sdt, \
+                 a.eps, (XT*)a.y, a.ldy, (const XT*)a.res, a.ldr);                                                   \
+    return true;                                                                                                     \
+  }
+  QTTS_WIDE(1, 1, 8, 2, 2)
+  QTTS_WIDE(1, 2, 8, 2, 2)
+  QTTS_WIDE(1, 3, 8, 2, 2)
+  QTTS_WIDE(1, 4, 8, 2, 2)
+  QTTS_WIDE(2, 2, 8, 2, 2)
+  QTTS_WIDE(2, 3, 8, 2, 2)
+  QTTS_WIDE(2, 4, 8, 2, 2)
+  if constexpr (!NORM) {
+    QTTS_WIDE(4, 3, 8, 2, 2)
+  }
+  QTTS_WIDE(1, 1, 16, 2, 2)
+  QTTS_WIDE(1, 2, 16, 2, 2)
+  QTTS_WIDE(1, 3, 16, 2, 2)
+  QTTS_WIDE(1, 4, 16, 2, 2)
+  if constexpr (!NORM) {
+    QTTS_WIDE(2, 2, 16, 2, 2)
+    QTTS_WIDE(2, 3, 16, 2, 2)
+    QTTS_WIDE(2, 4, 16, 2, 2)
+  }
+  QTTS_WIDE(1, 1, 8, 4, 4)
+  QTTS_WIDE(1, 2, 8, 4, 4)
+  if constexpr (!NORM) {
+    QTTS_WIDE(2, 2, 8, 4, 4)
+    QTTS_WIDE(1, 1, 8, 6, 6)
+    QTTS_WIDE(1, 2, 8, 6, 6)
+    QTTS_WIDE(1, 1, 16, 6, 4)
+    QTTS_WIDE(1, 2, 16, 6, 4)
+  }
+#undef QTTS_WIDE
+  return false;
+}
+
+}  // namespace qtts

@@ -1,0 +1,18 @@
+// The wide W8A16 kernel (wide.h), plain and with the residual add.
+#include "wide.h"
+
+using namespace qtts;
+
+// x [m, k] 16-bit, 16-byte aligned rows; strip weights; res [m, n] (row stride ldr) or NULL, may be y.
+// Returns QTTS_OK, 1 when the call is not this kernel's (wide_rule.h), or an error status.
+int qtts_launch_w8a16_wide(const void* x, int x_dtype, int64_t m, int64_t k, int64_t ldx, const int8_t* qs, int64_t n,
+                           const void* scale, int sdt, const void* bias, const void* res, int64_t ldr, void* y,
+                           int64_t ldy, hipStream_t st) {
+  const WideCfg c = wide_cfg(m, n, k);
+  if (c.mb == 0 || ldx > INT32_MAX) return 1;
+  const WideArgs a{x, m, ldx, qs, n, scale, sdt, bias, nullptr, 0.0f, res, ldr, y, ldy, st};
+  bool ok;
+  if (x_dtype == QTTS_BF16) ok = res ? launch_wide<bf16_t, kEpiRes, false, false>(c, a) : launch_wide<bf16_t, kEpiNone, false, false>(c, a);
+  else ok = res ? launch_wide<f16_t, kEpiRes, false, false>(c, a) : launch_wide<f16_t, kEpiNone, false, false>(c, a);
+  return ok ? qtts_check_launch("w8a16_wide") : 1;
+}

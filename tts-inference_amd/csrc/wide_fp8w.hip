@@ -1,0 +1,15 @@
+// The wide kernel (wide.h) on e4m3 codes: fp8 weight-only calls of 9 to 128 rows.
+#include "wide.h"
+
+using namespace qtts;
+
+// As qtts_launch_w8a16_wide, with fp32 scales and no residual.
+int qtts_launch_fp8w_wide(const void* x, int x_dtype, int64_t m, int64_t k, int64_t ldx, const uint8_t* qs, int64_t n,
+                          const float* scale, const void* bias, void* y, int64_t ldy, hipStream_t st) {
+  const WideCfg c = wide_cfg(m, n, k);
+  if (c.mb == 0 || ldx > INT32_MAX) return 1;
+  const WideArgs a{x, m, ldx, (const int8_t*)qs, n, scale, QTTS_F32, bias, nullptr, 0.0f, nullptr, 0, y, ldy, st};
+  const bool ok = x_dtype == QTTS_BF16 ? launch_wide<bf16_t, kEpiNone, false, true>(c, a)
+                                       : launch_wide<f16_t, kEpiNone, false, true>(c, a);
+  return ok ? qtts_check_launch("fp8w_wide") : 1;
+}

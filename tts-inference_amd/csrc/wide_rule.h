@@ -1,0 +1,62 @@
+// Which calls the wide kernel (wide.h) takes, and in which tile.
+#pragma once
+
+#include <stdint.h>
+
+namespace qtts {
+
+struct WideCfg { int mb, nb, waves, cpw; };  // mb == 0: not this kernel
+
+// The automatic choice for an [m, k] x [n, k] call, strip weights: 9 to 128 rows (8 and fewer stay with the
+// decode kernel, whose half strips and row staging are faster there; with the norm inside and K <= 1024 from 5
+// rows: 8 rows of the predictor's qkv 5.50 -> 5.00 us, of its gate_up with the activation 6.59 -> 5.65) where K is a built
+// product of waves and chunks and one of the built tiles covers the call in a single round of
+// workgroups on the 256 compute units.  Of those tiles the one that reads the fewest bytes a workgroup:
+// a second round costs more than any tile's extra bytes (the talker's gate_up past 32 rows, 512 workgroups,
+// 12.9 us at 48 rows against the tile kernel's 11.7).  K = 2048 runs 16 waves of 2 chunks on more than 128
+// strips and 8 of 4 on fewer (32 rows: talker qkv 4.49 against 4.84 us, o_proj + residual 4.43 against 4.19).
+// norm: with the RMSNorm inside, every workgroup repeats its rows' normalization, so the tile of the
+// fewest rows is taken and at most 32768 elements (16 rows of 2048): past them the norm's own launch
+// (about 2.7 us) is cheaper (talker gate_up at 32 rows 12.0 inside against 8.3 + 2.7; predictor gate_up
+// at 128 10.7 against 7.5 + 2.9, and inside up to 64 rows, 7.48 against 8.6).
+// pair: a gate_up weight with its activation.  K = 1024 past 48 rows: plain and residual calls stay with the
+// tile kernel, whose result the automatic choice is held to bit for bit there (they would
+// gain 0.1-0.9 us a call).
+inline WideCfg wide_cfg(int64_t m, int64_t n, int64_t k, bool norm = false, bool pair = false) {
+  WideCfg best{0, 0, 0, 0};
+  if (k == 1024 && m > 48 && !norm && !pair) return best;
+  if (m < (norm && k <= 1024 ? 5 : 9) || m > 128 || n <= 0 || n > (1 << 30)) return best;
+  const int64_t strips = (n + 15) / 16;
+  struct Tile { int mb, nb; };
+  static const Tile t82[] = {{1, 1}, {1, 2}, {1, 3}, {1, 4}, {2, 2}, {2, 3}, {2, 4}, {4, 3}};
+  static const Tile t162[] = {{1, 1}, {1, 2}, {1, 3}, {1, 4}, {2, 2}, {2, 3}, {2, 4}};
+  static const Tile t84[] = {{1, 1}, {1, 2}, {2, 2}};
+  static const Tile t86[] = {{1, 1}, {1, 2}};
+  const Tile* tiles;
+  int count, w, c;
+  switch (k) {
+    case 1024: tiles = t82, count = 8, w = 8, c = 2; break;
+    case 2048:
+      if (strips > 128) tiles = t162, count = 7, w = 16, c = 2;
+      else tiles = t84, count = 3, w = 8, c = 4;
+      break;
+    case 3072: tiles = t86, count = 2, w = 8, c = 6; break;
+    case 6144: tiles = t86, count = 2, w = 16, c = 6; break;
+    default: return best;
+  }
+  int64_t best_cost = 0;
+  for (int i = 0; i < count; ++i) {
+    const int mb = tiles[i].mb, nb = tiles[i].nb;
+    if (16 * mb >= m + 16) continue;  // a row block with no row of the call
+    if ((strips + nb - 1) / nb * ((m + 16 * mb - 1) / (16 * mb)) > 256) continue;
+    if (norm && (16 * mb * k > 32768 || k > 2048)) continue;
+    const int64_t cost = norm ? 8 * mb + nb : 2 * mb + nb;  // bytes a workgroup over 16 K
+    if (best.mb == 0 || cost < best_cost) {
+      best = WideCfg{mb, nb, w, c};
+      best_cost = cost;
+    }
+  }
+  return best;
+}
+
+}  // namespace qtts
