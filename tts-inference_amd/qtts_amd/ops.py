@@ -8,6 +8,7 @@ CPU or eager-PyTorch fallback: a missing library or an unsupported device raises
 
 from __future__ import annotations
 
+import functools
 import threading
 
 import torch
@@ -29,7 +30,10 @@ def dtype_code(dtype: torch.dtype) -> int:
 
 
 def _stream(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    """torch's current stream on ``device``, as the raw handle (building the Stream object that carries it
+    costs 1.8 us a call)."""
+    idx = device.index
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if idx is None else idx)
 
 
 def _ptr(t: torch.Tensor | None) -> int | None:
@@ -104,9 +108,16 @@ WORKSPACE_ROWS = 2048
 def reserve_for_rows(device: torch.device, op: int, n: int, k: int, max_rows: int = WORKSPACE_ROWS) -> None:
     """Reserve what ``op`` needs for an ``[N, K]`` weight at every row count up to ``max_rows``
     (the automatic kernel choice), outside capture: load time, not the hot path."""
+    reserve_workspace(device, _bytes_for_rows(op, n, k, int(max_rows)))
+
+
+@functools.lru_cache(maxsize=1024)
+def _bytes_for_rows(op: int, n: int, k: int, max_rows: int) -> int:
+    """The largest workspace ``op`` asks for up to ``max_rows`` rows: a function of the sizes alone, and a model's
+    layers share a few (12 queries of the library each time took a third of a layer's conversion)."""
     rows = sorted({r for r in (1, 2, 4, 8, 16, 32, 64, 128, 256, 512, 1024, 2048, 4096, 8192) if r <= max_rows}
-                  | {max(1, int(max_rows))})
-    reserve_workspace(device, max(workspace_bytes(op, r, n, k) for r in rows))
+                  | {max(1, max_rows)})
+    return max(workspace_bytes(op, r, n, k) for r in rows)
 
 
 def _ensure_workspace(device: torch.device, nbytes: int, what: str) -> None:
@@ -187,6 +198,8 @@ def pack_fp8(weight: torch.Tensor, div_mode: int = DIV_DEVICE):
 # ---- GEMMs --------------------------------------------------------------------------------
 
 def _flatten(x: torch.Tensor) -> torch.Tensor:
+    if x.dim() == 2 and x.stride(1) == 1 and (x.shape[0] <= 1 or x.stride(0) >= x.shape[1]):
+        return x
     rows = 1
     for d in x.shape[:-1]:
         rows *= d
@@ -194,6 +207,11 @@ def _flatten(x: torch.Tensor) -> torch.Tensor:
     if a.stride(-1) != 1 or (a.shape[0] > 1 and a.stride(0) < a.shape[1]):
         a = a.contiguous()
     return a
+
+
+def _shaped(out: torch.Tensor, shape: torch.Size) -> torch.Tensor:
+    """The ``[rows, n]`` output with the leading dimensions of the input's ``shape``."""
+    return out if len(shape) == 2 else out.reshape(*shape[:-1], out.shape[1])
 
 
 def w8a16_gemm(x: torch.Tensor, q: torch.Tensor, scale: torch.Tensor, bias: torch.Tensor | None = None,
@@ -229,7 +247,7 @@ def w8a16_gemm(x: torch.Tensor, q: torch.Tensor, scale: torch.Tensor, bias: torc
         _ptr(a), dtype_code(a.dtype), rows, k, a.stride(0) if rows > 1 else k, _ptr(q), n, q.stride(0),
         _ptr(scale), dtype_code(scale.dtype), _ptr(bias), _ptr(out), n, algo, ws, ws_n, _stream(dev))
     _lib.check(st, "w8a16_gemm")
-    return out.reshape(*shape[:-1], n)
+    return _shaped(out, shape)
 
 
 def quant_act_fp8(x: torch.Tensor, div_mode: int = DIV_DEVICE):
@@ -406,7 +424,7 @@ def w8a16_gemm_strips(x: torch.Tensor, qs: torch.Tensor, n: int, scale: torch.Te
         _ptr(a), dtype_code(a.dtype), rows, k, a.stride(0) if rows > 1 else k, _ptr(qs), n, _ptr(scale),
         dtype_code(scale.dtype), _ptr(bias), _ptr(out), n, algo, ws, ws_n, _stream(dev))
     _lib.check(st, "w8a16_gemm_strips")
-    return out.reshape(*shape[:-1], n)
+    return _shaped(out, shape)
 
 
 def w8a8_fp8_gemm_strips(qx: torch.Tensor, sx: torch.Tensor, qws: torch.Tensor, n: int, sw: torch.Tensor,
@@ -464,7 +482,7 @@ def fp8_linear_strips(x: torch.Tensor, qws: torch.Tensor, n: int, sw: torch.Tens
         _ptr(a), dtype_code(a.dtype), rows, k, a.stride(0) if rows > 1 else k, _ptr(qws), n, _ptr(sw), _ptr(bias),
         _ptr(out), n, div_mode, algo, ws, ws_n, _stream(dev))
     _lib.check(st, "fp8_linear_strips")
-    return out.reshape(*shape[:-1], n)
+    return _shaped(out, shape)
 
 
 # ---- int8 W8A8 (Int8Method, qtts/quant/int8.py:129-160) --------------------------------
@@ -575,7 +593,7 @@ def _int8_linear(x, qw, n, ldqw, sw, bias, div_mode, algo, strips):
             _ptr(a), dtype_code(a.dtype), rows, k, a.stride(0) if rows > 1 else k, _ptr(qw), n, ldqw, _ptr(sw),
             _ptr(bias), _ptr(out), n, div_mode, algo, ws, ws_n, _stream(dev))
     _lib.check(st, "int8_linear_strips" if strips else "int8_linear")
-    return out.reshape(*shape[:-1], n)
+    return _shaped(out, shape)
 
 
 def int8_linear(x: torch.Tensor, qw: torch.Tensor, sw: torch.Tensor, bias: torch.Tensor | None = None,
@@ -638,7 +656,7 @@ def fp8w_gemm_strips(x: torch.Tensor, qs: torch.Tensor, n: int, scale: torch.Ten
         _ptr(a), dtype_code(a.dtype), rows, k, a.stride(0) if rows > 1 else k, _ptr(qs), n, _ptr(scale), _ptr(bias),
         _ptr(out), n, algo, ws, ws_n, _stream(dev))
     _lib.check(st, "fp8w_gemm_strips")
-    return out.reshape(*shape[:-1], n)
+    return _shaped(out, shape)
 
 
 # ---- GatedMLP (qtts/layers/activation.py:142-147) ------------------------------------
@@ -690,7 +708,7 @@ def w8a16_silu_mul_gemm_strips(gate_up: torch.Tensor, qs: torch.Tensor, n: int, 
         _ptr(a), dtype_code(a.dtype), rows, k, a.stride(0) if rows > 1 else 2 * k, _ptr(qs), n, _ptr(scale),
         dtype_code(scale.dtype), _ptr(bias), _ptr(out), n, algo, ws, ws_n, _stream(dev))
     _lib.check(st, "w8a16_silu_mul_gemm_strips")
-    return out.reshape(*shape[:-1], n)
+    return _shaped(out, shape)
 
 
 def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float = 1e-6) -> torch.Tensor:
@@ -760,7 +778,7 @@ def w8a16_fused_gemm_strips(x: torch.Tensor, qs: torch.Tensor, n: int, scale: to
     _lib.check(st, "w8a16_fused_gemm_strips")
     if out is not None:
         return out
-    return y.reshape(*shape[:-1], n)
+    return _shaped(y, shape)
 
 
 def w8a16_gate_up_silu_strips(x: torch.Tensor, qs: torch.Tensor, n: int, scale: torch.Tensor,
@@ -800,7 +818,7 @@ def w8a16_gate_up_silu_strips(x: torch.Tensor, qs: torch.Tensor, n: int, scale: 
         float(eps), _ptr(qs), n, _ptr(scale), dtype_code(scale.dtype), _ptr(bias), _ptr(act), n // 2, algo, ws, ws_n,
         _stream(dev))
     _lib.check(st, "w8a16_gate_up_silu_strips")
-    return act.reshape(*shape[:-1], n // 2)
+    return _shaped(act, shape)
 
 
 class KernelTimer:
