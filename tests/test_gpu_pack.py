@@ -135,3 +135,46 @@ def test_pack_edge_shapes(ops):
         assert q.shape == (n, k)
         np.testing.assert_array_equal(q.cpu().numpy(), qo)
         np.testing.assert_array_equal(s32.cpu().numpy(), so)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("k", [8, 1016, 1024, 1032, 2048, 2056, 3072, 3080, 6144, 6152, 8192, 8200])
+def test_pack_vector_rows_equal_scalar_rows(ops, k, dtype):
+    """The packers' vector kernel (16-byte aligned rows) gives the scalar kernel's bytes and scales, at each of its
+    row lengths and the ones around them: ordinary rows, a zero row, one below the 1e-12 clamp, the type's
+    smallest and largest values, ties, an infinity and a NaN.  An odd row stride takes the scalar kernel."""
+    g = torch.Generator(device="cuda").manual_seed(k)
+    w = (torch.randn(11, k, device="cuda", generator=g) * 0.02).to(dtype)
+    w[1] = 0
+    w[2] = torch.finfo(dtype).smallest_normal if dtype == torch.bfloat16 else 0
+    w[3, ::3] = torch.finfo(dtype).tiny
+    w[4, -1] = torch.finfo(dtype).max
+    w[5] = (torch.arange(k, device="cuda") % 255 - 127).to(dtype) / 2
+    w[5, 0] = 127 if dtype == torch.float16 else 128
+    w[6, k // 2] = float("inf")
+    w[7, 0] = float("-inf")
+    w[8, k - 1] = float("nan")
+    odd = torch.empty(11, k + 1, device="cuda", dtype=dtype)[:, :k]
+    odd.copy_(w)
+    for mode in (ops.DIV_DEVICE, ops.DIV_IEEE):
+        for sdt in (torch.float32, dtype):
+            a, b = (ops.pack_int8(t, sdt, mode, want_f32_scale=True) for t in (w, odd))
+            assert torch.equal(a[0], b[0]) and all(torch.equal(p.view(torch.int32 if p.dtype == torch.float32 else torch.int16),
+                                                               q.view(torch.int32 if p.dtype == torch.float32 else torch.int16))
+                                                   for p, q in zip(a[1:], b[1:]))
+        a, b = (ops.pack_fp8(t, mode) for t in (w, odd))
+        assert torch.equal(a[0].view(torch.uint8), b[0].view(torch.uint8))
+        assert torch.equal(a[1].view(torch.int32), b[1].view(torch.int32))
+
+
+@pytest.mark.parametrize("n,k", [(16, 128), (33, 192), (5, 16), (48, 200)])
+def test_strips_round_trip_unaligned_rows(ops, n, k):
+    """Whole aligned slots (one 16-byte access) and ragged or unaligned ones: the same strips, and back."""
+    g = torch.Generator(device="cuda").manual_seed(n + k)
+    q = torch.randint(-127, 128, (n, k), device="cuda", generator=g, dtype=torch.int8)
+    odd = torch.empty(n, k + 1, device="cuda", dtype=torch.int8)[:, :k]
+    odd.copy_(q)
+    for kind in (ops.STRIP_INT8, ops.STRIP_FP8):
+        a = ops.to_strips(q, kind)
+        assert torch.equal(a.reshape(-1), ops.to_strips(odd, kind).reshape(-1))
+        assert torch.equal(ops.from_strips(a, n, k, kind), q)

@@ -1,5 +1,6 @@
 // Row-major <-> strip layout conversion (see layout.h).  Load-time only: one thread
-// per 16-byte lane slot, bounds-checked per byte at the ragged edges.
+// per 16-byte lane slot, one 16-byte access where the slot is whole and aligned, else
+// bounds-checked per byte.
 #include "common.h"
 #include "layout.h"
 
@@ -25,6 +26,11 @@ __global__ __launch_bounds__(256) void to_strips_kernel(const uint8_t* __restric
   const int64_t u = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (u >= units) return;
   const SlotPos p = slot_pos(u, nchunks, kind);
+  const uint8_t* from = src + p.row * ld + p.col;
+  if (p.row < n && p.col + 16 <= k && ((uintptr_t)from & 15) == 0) {  // a whole aligned slot: one load
+    *(uint4*)(dst + u * 16) = *(const uint4*)from;
+    return;
+  }
   uint8_t b[16];
 #pragma unroll
   for (int j = 0; j < 16; ++j) b[j] = (p.row < n && p.col + j < k) ? src[p.row * ld + p.col + j] : (uint8_t)0;
@@ -40,6 +46,11 @@ __global__ __launch_bounds__(256) void from_strips_kernel(const uint8_t* __restr
   if (u >= units) return;
   const SlotPos p = slot_pos(u, nchunks, kind);
   const uint4 v = *(const uint4*)(src + u * 16);
+  uint8_t* to = dst + p.row * ld + p.col;
+  if (p.row < n && p.col + 16 <= k && ((uintptr_t)to & 15) == 0) {
+    *(uint4*)to = v;
+    return;
+  }
   uint8_t b[16];
   __builtin_memcpy(b, &v, 16);
 #pragma unroll
