@@ -407,3 +407,24 @@ def test_int8_method_hook(ops):
         x = _acts(m, 2048, torch.bfloat16, seed=m + 7)
         q_t, s_t = _torch_act_int8(x)
         assert torch.equal(lin(x), _torch_int8_out(q_t, s_t, qw_ref, sw_ref, lin.bias, torch.bfloat16)), f"m={m}"
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("k", [8, 2048, 2056, 4096, 4104, 8192])
+def test_quant_act_int8_vector_rows_equal_scalar_rows(ops, k, dtype):
+    """The vector quantizer's quotients (row reciprocal, corrected) give the scalar kernel's codes and scales: ordinary
+    rows, ties, a zero row, one whose fp16 scale underflows, the largest value, an infinity and a NaN.  An odd row
+    stride takes the scalar kernel."""
+    g = torch.Generator(device="cuda").manual_seed(k)
+    x = (torch.randn(9, k, device="cuda", generator=g) * 3).to(dtype)
+    x[1] = 0
+    x[2] = 1e-7
+    x[3] = (torch.arange(k, device="cuda") % 255 - 127).to(dtype) / 2
+    x[4, k // 2] = torch.finfo(dtype).max
+    x[5, 0] = float("inf")
+    x[6, k - 1] = float("nan")
+    odd = torch.empty(9, k + 1, device="cuda", dtype=dtype)[:, :k]
+    odd.copy_(x)
+    for mode in (ops.DIV_DEVICE, ops.DIV_IEEE):
+        (a, sa), (b, sb) = ops.quant_act_int8(x, mode), ops.quant_act_int8(odd, mode)
+        assert torch.equal(a, b) and torch.equal(sa.view(torch.int32), sb.view(torch.int32))

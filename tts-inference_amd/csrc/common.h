@@ -281,9 +281,13 @@ template <typename XT> __device__ __forceinline__ float int8_act_scale(float ama
   return round_through<XT>(scalar_div(fmaxf(amax, round_through<XT>(1e-6f)), 127.0f, div_mode));
 }
 
-template <typename XT> __device__ __forceinline__ int int8_act_code(float x, float s) {
-  const float v = __builtin_rintf(round_through<XT>(x / s));
+__device__ __forceinline__ int int8_code_of(float quotient) {
+  const float v = __builtin_rintf(quotient);
   return v != v ? 0 : (int)fminf(fmaxf(v, -127.0f), 127.0f);
+}
+
+template <typename XT> __device__ __forceinline__ int int8_act_code(float x, float s) {
+  return int8_code_of(round_through<XT>(x / s));
 }
 
 // ---- wave64 reductions ----------------------------------------------------------------
