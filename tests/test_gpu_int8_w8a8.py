@@ -428,3 +428,32 @@ def test_quant_act_int8_vector_rows_equal_scalar_rows(ops, k, dtype):
     for mode in (ops.DIV_DEVICE, ops.DIV_IEEE):
         (a, sa), (b, sb) = ops.quant_act_int8(x, mode), ops.quant_act_int8(odd, mode)
         assert torch.equal(a, b) and torch.equal(sa.view(torch.int32), sb.view(torch.int32))
+
+
+# (m, n, k): every two-group tile of the automatic choice (128x128, 192x128, 128x192, 256x192 at these
+# sizes), one to many stages, ragged rows and columns
+TWO_GROUP = [(1500, 2048, 128), (2000, 1990, 256), (1500, 4096, 384), (1490, 4090, 128), (512, 12288, 256),
+             (1500, 12288, 128), (1024, 12288, 640), (1001, 12277, 512)]
+
+
+@pytest.mark.parametrize("out", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("m,n,k", TWO_GROUP)
+def test_two_group_tiles_equal_small_tiles(ops, m, n, k, out):
+    """int8: the automatic choice against a forced 64 x 128 tile, bit for bit (integer sums), with and without bias, a
+    strided activation matrix; fp8: the same K order, so the same bits there too."""
+    g = torch.Generator(device="cuda").manual_seed(m + n + k)
+    bias = torch.randn(n, device="cuda", generator=g).to(out)
+    sx = torch.rand(m, device="cuda", generator=g) + 0.5
+    sw = torch.rand(n, device="cuda", generator=g) + 0.5
+    forced = ops.algo_code(2, 1, 4, ops.tile_shape(64, 128, 8))
+    x = torch.randint(-127, 128, (m, k + 16), device="cuda", generator=g, dtype=torch.int8)[:, :k]
+    w = ops.to_strips(torch.randint(-127, 128, (n, k), device="cuda", generator=g, dtype=torch.int8))
+    for b in (None, bias):
+        assert torch.equal(ops.w8a8_int8_gemm_strips(x, sx, w, n, sw, b, out),
+                           ops.w8a8_int8_gemm_strips(x, sx, w, n, sw, b, out, forced))
+    xf = (torch.randn(m, k, device="cuda", generator=g) * 50).to(torch.float8_e4m3fn)
+    wf = ops.to_strips((torch.randn(n, k, device="cuda", generator=g) * 50).to(torch.float8_e4m3fn))
+    sx, sw = sx / 128, sw / 128  # fp16 outputs stay finite
+    for b in (None, bias):
+        assert torch.equal(ops.w8a8_fp8_gemm_strips(xf, sx, wf, n, sw, b, out),
+                           ops.w8a8_fp8_gemm_strips(xf, sx, wf, n, sw, b, out, forced))
