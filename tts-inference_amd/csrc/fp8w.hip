@@ -142,7 +142,7 @@ int64_t qtts_fp8w_ws_bytes(int64_t m, int64_t n, int64_t k, int algo) {
 int qtts_launch_fp8w(const void* x, int x_dtype, int64_t m, int64_t k, int64_t ldx, const uint8_t* qs, int64_t n,
                      const float* scale, const void* bias, void* y, int64_t ldy, int algo, void* ws, int64_t ws_bytes,
                      hipStream_t st) {
-  // 9 to 128 rows that one round of the wide kernel's workgroups covers (wide_rule.h)
+  // Up to 128 rows that one round of the wide kernels' workgroups covers (wide_rule.h)
   if (algo == QTTS_ALGO_AUTO) {
     const int rc = qtts_launch_fp8w_wide(x, x_dtype, m, k, ldx, qs, n, scale, bias, y, ldy, st);
     if (rc != 1) return rc;

@@ -299,7 +299,7 @@ static int launch_fast(const XT* x, int64_t m, int64_t k, int64_t ldx, const int
   int family = algo & 0xff;
   const int splits = (algo >> 8) & 0xff, waves = (algo >> 16) & 0xff;
   const bool wide_ok = LAYOUT == kLayoutStrips && k % 64 == 0;  // skinny beyond 16 rows
-  // 9 to 128 rows that one round of the wide kernel's workgroups covers (wide_rule.h)
+  // Up to 128 rows that one round of the wide kernels' workgroups covers (wide_rule.h)
   if (LAYOUT == kLayoutStrips && algo == QTTS_ALGO_AUTO) {
     const int rc = qtts_launch_w8a16_wide(x, std::is_same<XT, bf16_t>::value ? QTTS_BF16 : QTTS_F16, m, k, ldx, q, n,
                                           scale, sdt, bias, nullptr, 0, y, ldy, st);

@@ -452,7 +452,8 @@ int qtts_launch_w8a16_fused(const void* x, int x_dtype, int64_t m, int64_t k, in
     ldin = k;
   }
   // 3. The residual in the GEMM's epilogue (up to 16 staged rows, up to 64 on half strips).
-  const bool wide = kernel_ok && algo == QTTS_ALGO_AUTO && wide_cfg(m, n, k).mb > 0 && (uintptr_t)xin % 16 == 0 && ldin % 8 == 0;
+  const bool wide = kernel_ok && algo == QTTS_ALGO_AUTO && wide_takes(m, n, k) && (uintptr_t)xin % 16 == 0 &&
+                    (m == 1 || ldin % 8 == 0);
   if (res && wide && m <= 16) {
     const int rc = qtts_launch_w8a16_wide(xin, x_dtype, m, k, ldin, qs, n, scale, sdt, bias, res, ldr, y, ldy, st);
     if (rc != 1) return rc;

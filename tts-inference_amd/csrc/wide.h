@@ -47,8 +47,9 @@ __device__ __forceinline__ float add_row_lanes(float v) {
 // rounded as the reference rounds it (skinny.h: kProRmsNorm): each wave sums x^2 over its run, the
 // waves meet at one fence-free barrier while the weights stay in flight, and each scales its operands.
 // CL: chunks of a run that go through LDS; the rest load to registers in lane order (LDS holds no more).
-// (Weights load plainly under either weight policy: the streaming form measured 0.2-0.8 us a call slower.)
-template <typename XT, int MB, int NB, int W, int CPW, int CL, int EPI, bool NORM, bool F8W>
+// NT: the weight policy, as in skinny.h (alone, streaming loads measure 0.1-0.8 us a call slower; in a 12-layer
+// talker step they win, 32 rows 382.0 -> 379.0 us, 8 rows 289.2 -> 280.7 with the half strips below).
+template <typename XT, int MB, int NB, int W, int CPW, int CL, int EPI, bool NORM, bool F8W, bool NT>
 __global__ __launch_bounds__(W * 64) void w8a16_wide_kernel(
     const int8_t* __restrict__ qs, const XT* __restrict__ x, const void* scale, const XT* bias, const XT* aux, int ldx,
     int M, int N, int sdt, float eps, XT* y, int64_t ldy, const XT* res, int64_t ldr) {
@@ -102,7 +103,7 @@ __global__ __launch_bounds__(W * 64) void w8a16_wide_kernel(
       wp = qs + ((int64_t)s * nchunks + wc0) * 1024 + lane * 16;
     }
 #pragma unroll
-    for (int u = 0; u < CPW; ++u) w[u][nb] = load_weight<false>(wp + u * 1024);
+    for (int u = 0; u < CPW; ++u) w[u][nb] = load_weight<NT>(wp + u * 1024);
   }
   __builtin_amdgcn_sched_barrier(0);
 
@@ -261,6 +262,77 @@ __global__ __launch_bounds__(W * 64) void w8a16_wide_kernel(
   }
 }
 
+// The same for up to 8 rows a workgroup on few strips: a workgroup takes half a strip (8 weight rows) of one
+// 8-row part of the call, so 64 or 128 strips still spread over the GPU.  One MFMA covers two chunks ("a unit"), as
+// skinny.h's half strips: A rows 0-7 and B columns 0-7 hold the even chunk, rows 8-15 and columns 8-15 the odd
+// one, and the two diagonal blocks of D are added in the epilogue.  K = 128 W UPW.  What it has over the half strips
+// of skinny.h: the rows go straight to LDS (no registers, no LDS writes) and 8-12 waves share a row's loads.
+// Measured as above, us a call, skinny.h's half strips (9-16 rows: the kernel above) -> this one, with the
+// residual add, at 4 / 8 / 16 rows: the talker's o_proj 3.39 / 3.51 -> 3.21 / 3.23 at 4 / 8, its down_proj 5.19 / 6.11 ->
+// 4.73 / 4.62; the predictor's o_proj 4.15 / 4.37 / 4.60 -> 3.88 / 3.92 / 4.07, its down_proj 4.60 / 5.07 / 5.02 ->
+// 4.15 / 4.14 / 4.35; its 1-stream frame 1243 -> 1158.
+template <typename XT, int W, int UPW, int EPI, bool F8W, bool NT>
+__global__ __launch_bounds__(W * 64) void w8a16_wide_half_kernel(
+    const int8_t* __restrict__ qs, const XT* __restrict__ x, const void* scale, const XT* bias, int ldx, int M, int N, int sdt,
+    XT* y, int64_t ldy, const XT* res, int64_t ldr) {
+  typedef mfma16<XT> MM;
+  typedef typename MM::vec V;
+  constexpr int P = 16 * UPW, XI = 2 * UPW, nchunks = 2 * W * UPW;
+  __shared__ __align__(1024) uint8_t lds[W][XI * 1024];
+  const int strip = blockIdx.x >> 1, part = (blockIdx.x & 1) * 8, y0 = blockIdx.z * 8;
+  if (strip * 16 + part >= N) return;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r = lane & 15, g = lane >> 4;
+  const int u0 = wave * UPW;
+#pragma unroll
+  for (int i = 0; i < XI; ++i) {
+    const int flat = i * 64 + lane, row = flat / P, p = flat % P;
+    load_to_lds16(x + (int64_t)min(y0 + row, M - 1) * ldx + u0 * 128 + 8 * (p ^ row), &lds[wave][i * 1024]);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  i32x4_t w[UPW];
+  const int8_t* wp = qs + ((int64_t)strip * nchunks + 2 * u0 + (r >> 3)) * 1024 + (part + (r & 7) + 16 * g) * 16;
+#pragma unroll
+  for (int u = 0; u < UPW; ++u) w[u] = load_weight<NT>(wp + u * 2048);
+  __builtin_amdgcn_sched_barrier(0);
+  // output (row m, column n) of lane: n = lane % 8, m = lane / 8
+  const int on = min(strip * 16 + part + (lane & 7), N - 1), om = min(y0 + (lane >> 3), M - 1);
+  const uint32_t sc = load_scale_bits(scale, sdt, on);
+  const uint32_t bi = load_bits((bias ? bias : x) + (bias ? on : 0));
+  uint32_t rb = 0;
+  if constexpr (EPI == kEpiRes) rb = load_bits(res + (int64_t)om * ldr + on);
+  __builtin_amdgcn_sched_barrier(0);
+  wait_vmcnt<UPW>();
+  V xa[UPW], xb[UPW];
+#pragma unroll
+  for (int u = 0; u < UPW; ++u) {
+    const int row = r & 7, p = 16 * u + 8 * (r >> 3) + 2 * g;
+    xa[u] = *(const V*)&lds[wave][(row * P + (p ^ row)) * 16];
+    xb[u] = *(const V*)&lds[wave][(row * P + ((p + 1) ^ row)) * 16];
+  }
+  f32x4_t acc = {0, 0, 0, 0};
+#pragma unroll
+  for (int u = 0; u < UPW; ++u) {
+    acc = MM::mma(wcvt<F8W, XT>((uint32_t)w[u][0], (uint32_t)w[u][1]), xa[u], acc);
+    acc = MM::mma(wcvt<F8W, XT>((uint32_t)w[u][2], (uint32_t)w[u][3]), xb[u], acc);
+  }
+  *(f32x4_t*)&lds[wave][lane * 16] = acc;
+  __syncthreads();
+  if (wave > 0) return;
+  const int n = lane & 7, m = lane >> 3;
+  const int src = (m + 16 * (n >> 2)) * 16 + 4 * (n & 3), src2 = ((m + 16 * (n >> 2)) ^ 40) * 16 + 4 * (n & 3);
+  float a = 0.0f, b = 0.0f;
+#pragma unroll
+  for (int v = 0; v < W; ++v) {
+    a += *(const float*)&lds[v][src];
+    b += *(const float*)&lds[v][src2];
+  }
+  float f = (a + b) * scale_bits_to_f32(sc, sdt);
+  if (bias) f += xbits_to_f32<XT>(bi);
+  if constexpr (EPI == kEpiRes) f = xbits_to_f32<XT>(rb) + round_through<XT>(f);
+  if (y0 + m < M && strip * 16 + part + n < N) y[(int64_t)(y0 + m) * ldy + strip * 16 + part + n] = from_f32<XT>(f);
+}
+
 struct WideArgs {
   const void* x; int64_t m, ldx; const int8_t* qs; int64_t n; const void* scale; int sdt; const void* bias;
   const void* aux; float eps; const void* res; int64_t ldr; void* y; int64_t ldy; hipStream_t st;
@@ -272,9 +344,11 @@ template <typename XT, int EPI, bool NORM, bool F8W> inline bool launch_wide(con
   const dim3 grid((unsigned)(((strips + c.nb - 1) / c.nb + 7) / 8 * 8), 1, (unsigned)((a.m + 16 * c.mb - 1) / (16 * c.mb)));
 #define QTTS_WIDE(MB, NB, W, CPW, CL)                                                                                \
   if (c.mb == MB && c.nb == NB && c.waves == W && c.cpw == CPW) {                                                    \
-    qtts::launch(&w8a16_wide_kernel<XT, MB, NB, W, CPW, CL, EPI, NORM, F8W>, grid, dim3(W * 64), 0, a.st, a.qs,      \
-                 (const XT*)a.x, a.scale, (const XT*)a.bias, (const XT*)a.aux, (int)a.ldx, (int)a.m, (int)a.n, a.sdt, \
-                 a.eps, (XT*)a.y, a.ldy, (const XT*)a.res, a.ldr);                                                   \
+    qtts::launch_by_policy<std::is_same<XT, bf16_t>::value>([&](auto nt) {                                           \
+      qtts::launch(&w8a16_wide_kernel<XT, MB, NB, W, CPW, CL, EPI, NORM, F8W, decltype(nt)::value>, grid,            \
+                   dim3(W * 64), 0, a.st, a.qs, (const XT*)a.x, a.scale, (const XT*)a.bias, (const XT*)a.aux,        \
+                   (int)a.ldx, (int)a.m, (int)a.n, a.sdt, a.eps, (XT*)a.y, a.ldy, (const XT*)a.res, a.ldr);          \
+    });                                                                                                              \
     return true;                                                                                                     \
   }
   QTTS_WIDE(1, 1, 8, 2, 2)
@@ -306,6 +380,25 @@ template <typename XT, int EPI, bool NORM, bool F8W> inline bool launch_wide(con
     QTTS_WIDE(1, 2, 16, 6, 4)
   }
 #undef QTTS_WIDE
+  return false;
+}
+
+// One launch of a configuration of half_cfg (wide_rule.h).
+template <typename XT, int EPI, bool F8W> inline bool launch_half(const HalfCfg& c, const WideArgs& a) {
+  const dim3 grid((unsigned)((a.n + 15) / 16 * 2), 1, (unsigned)((a.m + 7) / 8));
+#define QTTS_HALF(W, UPW)                                                                                       \
+  if (c.waves == W && c.upw == UPW) {                                                                           \
+    qtts::launch_by_policy<std::is_same<XT, bf16_t>::value>([&](auto nt) {                                      \
+      qtts::launch(&w8a16_wide_half_kernel<XT, W, UPW, EPI, F8W, decltype(nt)::value>, grid, dim3(W * 64), 0, a.st, \
+                   a.qs, (const XT*)a.x, a.scale, (const XT*)a.bias, (int)a.ldx, (int)a.m, (int)a.n, a.sdt,     \
+                   (XT*)a.y, a.ldy, (const XT*)a.res, a.ldr);                                                   \
+    });                                                                                                         \
+    return true;                                                                                                \
+  }
+  QTTS_HALF(8, 2)
+  QTTS_HALF(8, 3)
+  QTTS_HALF(12, 4)
+#undef QTTS_HALF
   return false;
 }
 

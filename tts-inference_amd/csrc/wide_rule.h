@@ -59,4 +59,22 @@ inline WideCfg wide_cfg(int64_t m, int64_t n, int64_t k, bool norm = false, bool
   return best;
 }
 
+struct HalfCfg { int waves, upw; };  // waves == 0: not this kernel
+
+// Half strips in 8-row parts (wide.h): where the strips times two times the parts make one round of at most 256
+// workgroups (up to 16 rows on 64 strips, 8 on 128) and K is a built product.  From 2 rows: at one row the
+// staged rows are few and the 28-layer talker step ran 511.5 us with these against 509.2 without.
+inline HalfCfg half_cfg(int64_t m, int64_t n, int64_t k) {
+  if (m < 2 || n < 1 || (n + 15) / 16 * 2 * ((m + 7) / 8) > 256) return HalfCfg{0, 0};
+  if (k == 2048) return HalfCfg{8, 2};
+  if (k == 3072) return HalfCfg{8, 3};
+  if (k == 6144) return HalfCfg{12, 4};
+  return HalfCfg{0, 0};
+}
+
+// Whether the automatic choice runs a plain (or residual) call on the wide kernels.
+inline bool wide_takes(int64_t m, int64_t n, int64_t k) {
+  return half_cfg(m, n, k).waves > 0 || wide_cfg(m, n, k).mb > 0;
+}
+
 }  // namespace qtts
