@@ -268,9 +268,8 @@ __global__ __launch_bounds__(W * 64) void w8a16_wide_kernel(
 // one, and the two diagonal blocks of D are added in the epilogue.  K = 128 W UPW.  What it has over the half strips
 // of skinny.h: the rows go straight to LDS (no registers, no LDS writes) and 8-12 waves share a row's loads.
 // Measured as above, us a call, skinny.h's half strips (9-16 rows: the kernel above) -> this one, with the
-// residual add, at 4 / 8 / 16 rows: the talker's o_proj 3.39 / 3.51 -> 3.21 / 3.23 at 4 / 8, its down_proj 5.19 / 6.11 ->
-// 4.73 / 4.62; the predictor's o_proj 4.15 / 4.37 / 4.60 -> 3.88 / 3.92 / 4.07, its down_proj 4.60 / 5.07 / 5.02 ->
-// 4.15 / 4.14 / 4.35; its 1-stream frame 1243 -> 1158.
+// residual add, at 8 / 16 rows: the talker's o_proj 3.51 -> 3.23 at 8, its down_proj 6.11 -> 4.62; the predictor's
+// o_proj 4.37 / 4.60 -> 3.92 / 4.07, its down_proj 5.07 / 5.02 -> 4.14 / 4.35; its 1-stream frame 1243 -> 1158.
 template <typename XT, int W, int UPW, int EPI, bool F8W, bool NT>
 __global__ __launch_bounds__(W * 64) void w8a16_wide_half_kernel(
     const int8_t* __restrict__ qs, const XT* __restrict__ x, const void* scale, const XT* bias, int ldx, int M, int N, int sdt,

@@ -62,10 +62,12 @@ inline WideCfg wide_cfg(int64_t m, int64_t n, int64_t k, bool norm = false, bool
 struct HalfCfg { int waves, upw; };  // waves == 0: not this kernel
 
 // Half strips in 8-row parts (wide.h): where the strips times two times the parts make one round of at most 256
-// workgroups (up to 16 rows on 64 strips, 8 on 128) and K is a built product.  From 2 rows: at one row the
-// staged rows are few and the 28-layer talker step ran 511.5 us with these against 509.2 without.
+// workgroups (up to 16 rows on 64 strips, 8 on 128) and K is a built product.  From 5 rows: below,
+// skinny.h stages fewer rows, and whole steps run faster on it: 10 predictor layers at 2 / 4 rows 155.1 / 165.3 us
+// against 160.7 / 167.9 with these (8 rows: 187.1 against 177.9), 4 talker layers 85.9 / 91.6 against 87.6 / 92.0
+// (8 rows: 107.0 against 103.0).
 inline HalfCfg half_cfg(int64_t m, int64_t n, int64_t k) {
-  if (m < 2 || n < 1 || (n + 15) / 16 * 2 * ((m + 7) / 8) > 256) return HalfCfg{0, 0};
+  if (m < 5 || n < 1 || (n + 15) / 16 * 2 * ((m + 7) / 8) > 256) return HalfCfg{0, 0};
   if (k == 2048) return HalfCfg{8, 2};
   if (k == 3072) return HalfCfg{8, 3};
   if (k == 6144) return HalfCfg{12, 4};
