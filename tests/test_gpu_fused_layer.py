@@ -238,6 +238,46 @@ def test_fused_errors(ops):
     assert st != 0 and "prologue" in _lib.last_error()
 
 
+@pytest.mark.parametrize("m,n,k", [(8, 2048, 2048), (16, 1024, 3072), (17, 2048, 2048), (40, 2048, 2048), (41, 2048, 2048),
+                                   (64, 1024, 2048), (65, 1024, 2048)])
+def test_residual_without_a_workspace(ops, m, n, k):
+    """A residual call that the decode kernels' half strips cover (up to 64 rows, their weight reads within 20 MiB) runs
+    without a workspace and gives the bits it gives with one, whichever kernel the automatic choice takes; past
+    them the call is refused."""
+    from qtts_amd import _lib
+    q, s, qs = _weights(ops, n, k, torch.bfloat16, 9)
+    g = torch.Generator(device="cuda").manual_seed(m)
+    x = torch.randn(m, k, device="cuda", generator=g).to(torch.bfloat16)
+    res = torch.randn(m, n, device="cuda", generator=g).to(torch.bfloat16)
+    y = torch.empty_like(res)
+    st = _lib.load().qtts_w8a16_fused_gemm_strips(
+        x.data_ptr(), _lib.BF16, m, k, k, ops.PRO_NONE, None, 0.0, qs.data_ptr(), n, s.data_ptr(), _lib.BF16, None,
+        res.data_ptr(), n, y.data_ptr(), n, 0, None, 0, torch.cuda.current_stream().cuda_stream)
+    if m <= 16 or (m <= 64 and (m + 7) // 8 * n * k <= 20 << 20):
+        assert st == 0, _lib.last_error()
+        assert torch.equal(y, ops.w8a16_fused_gemm_strips(x, qs, n, s, residual=res))
+    else:
+        assert st != 0 and "workspace" in _lib.last_error()
+
+
+@pytest.mark.parametrize("m,n,k", [(12, 512, 4096), (12, 512, 6144), (17, 512, 2048)])
+def test_gate_up_without_a_workspace(ops, m, n, k):
+    """gate_up with its activation needs no workspace where the decode kernel's pairs are built (16 rows, K <= 4096);
+    elsewhere a call that comes without is refused, whichever kernel would run it."""
+    from qtts_amd import _lib
+    q, s, qs = _weights(ops, n, k, torch.bfloat16, 9)
+    x = torch.randn(m, k, device="cuda").to(torch.bfloat16)
+    act = torch.empty(m, n // 2, device="cuda", dtype=torch.bfloat16)
+    st = _lib.load().qtts_w8a16_gate_up_silu_strips(
+        x.data_ptr(), _lib.BF16, m, k, k, ops.PRO_NONE, None, 0.0, qs.data_ptr(), n, s.data_ptr(), _lib.BF16, None,
+        act.data_ptr(), n // 2, 0, None, 0, torch.cuda.current_stream().cuda_stream)
+    if m <= 16 and k <= 4096:
+        assert st == 0, _lib.last_error()
+        assert torch.equal(act, ops.w8a16_gate_up_silu_strips(x, qs, n, s))
+    else:
+        assert st != 0 and "workspace" in _lib.last_error()
+
+
 # (m, n, k): tiles of 32 x 64 with one and two chunks a stage, whole and split K, ragged rows and
 # columns; then each 8-wave tile of the automatic choice.
 TILE_EPILOGUES = [(65, 100, 192), (17, 4128, 64), (70, 2048, 6144), (129, 1056, 1024), (1003, 2048, 128),

@@ -241,6 +241,76 @@ int64_t qtts_w8a16_fused_ws_bytes(int64_t m, int64_t n, int64_t k, int algo, int
 
 namespace {
 
+// The row split, configuration and grid of one fused launch (not a pair), into a: QTTS_OK, 1 when no built form takes the call
+// (the caller then runs the separate kernels), or an error status.
+int plan_fused(int pro, int algo, void* ws, int64_t ws_bytes, FusedArgs& a) {
+  const int splits = (algo >> 8) & 0xff, waves = (algo >> 16) & 0xff, cpw = (algo >> 24) & 0x3f;
+  const int64_t m = a.m, n = a.n, k = a.k;
+  // Row-split strips: the plain launch's choice (w8a16.hip launch_fast), so a fused call and the
+  // plain GEMM it replaces give the same bits.
+  const int family = algo & 0xff;
+  int sub = family == QTTS_ALGO_SKINNY_HALF ? 2 : (family == QTTS_ALGO_SKINNY_QUARTER ? 4 : 1);
+  if (sub > 1 && (splits != 0 || !skinny_sub_rows_ok(m, k, sub))) return 1;  // the separate path reports it
+  if (family == QTTS_ALGO_AUTO && splits == 0 && (algo >> 16) == 0)
+    sub = m <= 8 ? skinny_auto_sub(m, n, k) : skinny_row_parts_sub(m, n, k);
+  // Up to 16 rows (9-16 in two row parts of 8); past 16 only on half strips in row parts, where
+  // the plain GEMM takes them too.
+  if (m > 16 && sub != 2) return 1;
+  a.sub = sub;
+  a.counters = nullptr;
+  a.part = nullptr;
+  if (sub > 1) {
+    a.c = skinny_cfg_sub(n, k, sub, waves, cpw);
+    if (pro == kProRmsNorm || !fused_sub_built(sub, a.c.waves, a.c.cpw) || a.c.waves * a.c.cpw < a.c.cps || a.ldx > INT32_MAX)
+      return 1;
+    a.blocks = (unsigned)(((int64_t)a.c.strips * sub + 7) / 8 * 8);
+    return QTTS_OK;
+  }
+  SkinnyCfg c = skinny_cfg(m, n, k, splits, waves, cpw);
+  // As the plain staged launch: 8 waves of 12 chunks from 2 to 8 rows for long K.
+  if (m >= 2 && m <= 8 && waves == 0 && cpw == 0 && c.waves == 16 && c.S == 1 && 8 * 12 >= (k + 63) / 64)
+    c = skinny_cfg(m, n, k, splits, 8, 12);
+  const int64_t need = skinny_ws(c);
+  if (need > ws_bytes || (need > 0 && !ws)) {
+    if (splits > 0)
+      return qtts_set_error(QTTS_ERR_WORKSPACE, "w8a16 fused: %d splits need %lld workspace bytes, got %lld", c.S,
+                            (long long)need, (long long)ws_bytes);
+    c = skinny_cfg(m, n, k, 1, 16, 6);  // no room for a split: longer runs per wave
+    if (c.S > 1) return 1;
+  }
+  if (!qtts_w8a16_xrows_built(c.waves, c.cpw)) return 1;
+  if ((pro == kProRmsNorm || m > 8) && c.S > 1) return 1;  // row parts need one split
+  if (c.S > 1 && c.strips > kMaxSplitTiles) return 1;
+  if (c.S > 65535) return 1;  // past the grid's y limit
+  const int64_t blocks = (int64_t)((c.strips + 7) / 8) * 8;  // grid x; grid y: the K splits
+  if (blocks >= ((int64_t)1 << 31) || a.ldx > INT32_MAX) return 1;
+  a.c = c;
+  a.blocks = (unsigned)blocks;
+  a.counters = (unsigned*)ws;
+  a.part = ws ? (float*)((char*)ws + kCounterBytes) : nullptr;
+  return QTTS_OK;
+}
+
+// Launches a planned call: QTTS_OK, 1 when its variant is not built, or an error status.
+int launch_plan(int pro, bool res, const FusedArgs& a, int x_dtype, int sdt) {
+  const bool f32s = sdt == QTTS_F32;
+  const int64_t m = a.m;
+  int rc = 1;
+  if (pro == kProSiluMul) rc = res ? launch_fused<kProSiluMul, true, 1>(x_dtype, f32s, a)
+                                   : launch_fused<kProSiluMul, false, 1>(x_dtype, f32s, a);
+  else if (pro == kProRmsNorm && !res)
+    rc = m == 1 ? launch_fused<kProRmsNorm, false, 1>(x_dtype, f32s, a)
+                : m == 2 ? launch_fused<kProRmsNorm, false, 2>(x_dtype, f32s, a)
+                : (m <= 4 ? launch_fused<kProRmsNorm, false, 4>(x_dtype, f32s, a)
+                          : launch_fused<kProRmsNorm, false, 8>(x_dtype, f32s, a));
+  else if (pro == kProNone && res)
+    rc = m == 1 ? launch_fused<kProNone, true, 1>(x_dtype, f32s, a)
+                : m == 2 ? launch_fused<kProNone, true, 2>(x_dtype, f32s, a)
+                : (m <= 4 ? launch_fused<kProNone, true, 4>(x_dtype, f32s, a) : launch_fused<kProNone, true, 8>(x_dtype, f32s, a));
+  if (rc != 0) return 1;
+  return qtts_check_launch(a.sub > 1 ? "w8a16_fused_skinny_sub" : "w8a16_fused_skinny");
+}
+
 // One fused skinny launch: QTTS_OK, 1 when this call cannot be fused (the caller then
 // runs the separate kernels), or an error status.  pair: the SiLU-pair gate_up launch
 // (in.n is the fused gate_up width; one workgroup per gate strip, no split).
@@ -317,75 +387,9 @@ int try_fused(int pro, bool res, const FusedArgs& in, int x_dtype, int sdt, int 
     if (rc != 0) return 1;
     return qtts_check_launch("w8a16_gate_up_silu");
   }
-  // Row-split strips: the plain launch's choice (w8a16.hip launch_fast), so a fused call and the
-  // plain GEMM it replaces give the same bits.
-  const int family = algo & 0xff;
-  int sub = family == QTTS_ALGO_SKINNY_HALF ? 2 : (family == QTTS_ALGO_SKINNY_QUARTER ? 4 : 1);
-  if (sub > 1 && (splits != 0 || !skinny_sub_rows_ok(m, k, sub))) return 1;  // the separate path reports it
-  if (family == QTTS_ALGO_AUTO && splits == 0 && (algo >> 16) == 0)
-    sub = m <= 8 ? skinny_auto_sub(m, n, k) : skinny_row_parts_sub(m, n, k);
-  // Up to 16 rows (9-16 in two row parts of 8); past 16 only on half strips in row parts, where
-  // the plain GEMM takes them too.
-  if (m > 16 && sub != 2) return 1;
-  if (sub > 1) {
-    const SkinnyCfg c = skinny_cfg_sub(n, k, sub, waves, cpw);
-    if (!fused_sub_built(sub, c.waves, c.cpw) || c.waves * c.cpw < c.cps || in.ldx > INT32_MAX) return 1;
-    FusedArgs a = in;
-    a.c = c;
-    a.sub = sub;
-    a.blocks = (unsigned)(((int64_t)c.strips * sub + 7) / 8 * 8);
-    a.counters = nullptr;
-    a.part = nullptr;
-    const bool f32s = sdt == QTTS_F32;
-    int rc = 1;
-    if (pro == kProSiluMul) rc = res ? launch_fused<kProSiluMul, true, 1>(x_dtype, f32s, a)
-                                     : launch_fused<kProSiluMul, false, 1>(x_dtype, f32s, a);
-    else if (pro == kProNone && res)
-      rc = m == 1 ? launch_fused<kProNone, true, 1>(x_dtype, f32s, a)
-                  : m == 2 ? launch_fused<kProNone, true, 2>(x_dtype, f32s, a)
-                  : (m <= 4 ? launch_fused<kProNone, true, 4>(x_dtype, f32s, a)
-                            : launch_fused<kProNone, true, 8>(x_dtype, f32s, a));
-    if (rc != 0) return 1;
-    return qtts_check_launch("w8a16_fused_skinny_sub");
-  }
-  SkinnyCfg c = skinny_cfg(m, n, k, splits, waves, cpw);
-  // As the plain staged launch: 8 waves of 12 chunks from 2 to 8 rows for long K.
-  if (m >= 2 && m <= 8 && waves == 0 && cpw == 0 && c.waves == 16 && c.S == 1 && 8 * 12 >= (k + 63) / 64)
-    c = skinny_cfg(m, n, k, splits, 8, 12);
-  const int64_t need = skinny_ws(c);
-  if (need > ws_bytes || (need > 0 && !ws)) {
-    if (splits > 0)
-      return qtts_set_error(QTTS_ERR_WORKSPACE, "w8a16 fused: %d splits need %lld workspace bytes, got %lld", c.S,
-                            (long long)need, (long long)ws_bytes);
-    c = skinny_cfg(m, n, k, 1, 16, 6);  // no room for a split: longer runs per wave
-    if (c.S > 1) return 1;
-  }
-  if (!qtts_w8a16_xrows_built(c.waves, c.cpw)) return 1;
-  if ((pro == kProRmsNorm || m > 8) && c.S > 1) return 1;  // row parts need one split
-  if (c.S > 1 && c.strips > kMaxSplitTiles) return 1;
-  if (c.S > 65535) return 1;  // past the grid's y limit
-  const int64_t blocks = (int64_t)((c.strips + 7) / 8) * 8;  // grid x; grid y: the K splits
-  if (blocks >= ((int64_t)1 << 31) || in.ldx > INT32_MAX) return 1;
   FusedArgs a = in;
-  a.c = c;
-  a.blocks = (unsigned)blocks;
-  a.counters = (unsigned*)ws;
-  a.part = ws ? (float*)((char*)ws + kCounterBytes) : nullptr;
-  const bool f32s = sdt == QTTS_F32;
-  int rc = 1;
-  if (pro == kProSiluMul) rc = res ? launch_fused<kProSiluMul, true, 1>(x_dtype, f32s, a)
-                                   : launch_fused<kProSiluMul, false, 1>(x_dtype, f32s, a);
-  else if (pro == kProRmsNorm && !res)
-    rc = m == 1 ? launch_fused<kProRmsNorm, false, 1>(x_dtype, f32s, a)
-                : m == 2 ? launch_fused<kProRmsNorm, false, 2>(x_dtype, f32s, a)
-                : (m <= 4 ? launch_fused<kProRmsNorm, false, 4>(x_dtype, f32s, a)
-                          : launch_fused<kProRmsNorm, false, 8>(x_dtype, f32s, a));
-  else if (pro == kProNone && res)
-    rc = m == 1 ? launch_fused<kProNone, true, 1>(x_dtype, f32s, a)
-                : m == 2 ? launch_fused<kProNone, true, 2>(x_dtype, f32s, a)
-                : (m <= 4 ? launch_fused<kProNone, true, 4>(x_dtype, f32s, a) : launch_fused<kProNone, true, 8>(x_dtype, f32s, a));
-  if (rc != 0) return 1;
-  return qtts_check_launch("w8a16_fused_skinny");
+  const int rc = plan_fused(pro, algo, ws, ws_bytes, a);
+  return rc == QTTS_OK ? launch_plan(pro, res, a, x_dtype, sdt) : rc;
 }
 
 }  // namespace
@@ -452,16 +456,18 @@ int qtts_launch_w8a16_fused(const void* x, int x_dtype, int64_t m, int64_t k, in
     ldin = k;
   }
   // 3. The residual in the GEMM's epilogue (up to 16 staged rows, up to 64 on half strips).
-  const bool wide = kernel_ok && algo == QTTS_ALGO_AUTO && wide_takes(m, n, k) && (uintptr_t)xin % 16 == 0 &&
-                    (m == 1 || ldin % 8 == 0);
-  if (res && wide && m <= 16) {
-    const int rc = qtts_launch_w8a16_wide(xin, x_dtype, m, k, ldin, qs, n, scale, sdt, bias, res, ldr, y, ldy, st);
-    if (rc != 1) return rc;
-  }
-  if (res && kernel_ok && !wide && m <= kRowPartsMaxM && (uintptr_t)xin % 16 == 0 && (m == 1 || ldin % 8 == 0)) {
+  // The wide kernels need no workspace, but take only the calls that bring what they must without them: the
+  // decode forms' (plan_fused: none), or the separate kernels' below.
+  const bool xin_aligned = (uintptr_t)xin % 16 == 0 && (m == 1 || ldin % 8 == 0);
+  const bool wide = kernel_ok && algo == QTTS_ALGO_AUTO && wide_takes(m, n, k) && xin_aligned;
+  if (res && kernel_ok && m <= kRowPartsMaxM && xin_aligned) {
     a.x = xin;
     a.ldx = ldin;
-    const int rc = try_fused(kProNone, true, a, x_dtype, sdt, algo, ws, avail);
+    int rc = plan_fused(kProNone, algo, ws, avail, a);
+    if (rc == QTTS_OK) {
+      rc = wide ? qtts_launch_w8a16_wide(xin, x_dtype, m, k, ldin, qs, n, scale, sdt, bias, res, ldr, y, ldy, st) : 1;
+      if (rc == 1) rc = launch_plan(kProNone, true, a, x_dtype, sdt);
+    }
     if (rc != 1) return rc;
   }
   // 4. The plain GEMM, then the residual (the GEMM writes into the workspace: y may be
@@ -521,7 +527,8 @@ int qtts_launch_w8a16_gate_up_silu(const void* x, int x_dtype, int64_t m, int64_
                          family != QTTS_ALGO_TILE && !direct_x;
   const bool x_aligned = (uintptr_t)x % 16 == 0 && (m == 1 || ldx % 8 == 0);
   const bool wide_pair = kernel_ok && x_aligned && algo == QTTS_ALGO_AUTO && n % 32 == 0 && ldx % 8 == 0;
-  if (wide_pair && m <= 16 && (pro == kProNone || (uintptr_t)nw % 16 == 0)) {
+  // Up to 16 rows of K <= 4096 the decode kernel's pairs are built and need no workspace, so these calls may come without.
+  if (wide_pair && m <= 16 && k <= 4096 && (pro == kProNone || (uintptr_t)nw % 16 == 0)) {
     const int rc = qtts_launch_w8a16_wide_fused(x, x_dtype, m, k, ldx, pro == kProNone ? nullptr : nw, eps, qs, n, scale, sdt,
                                                 bias, true, act, ldact, st);
     if (rc != 1) return rc;
@@ -553,7 +560,11 @@ int qtts_launch_w8a16_gate_up_silu(const void* x, int x_dtype, int64_t m, int64_
   const int64_t avail = (ws_bytes - g_bytes) & ~(int64_t)255;
   void* gu = (char*)ws + avail;
   // Past the decode rows: one wide launch with the norm and the activation, or the norm, then one wide or
-  // tile launch with the activation in its epilogue.
+  // tile launch with the activation in its epilogue.  Below them, what the wide kernel takes of the longer K.
+  if (wide_pair && m <= 16 && k > 4096 && pro == kProNone) {
+    const int rc = qtts_launch_w8a16_wide_fused(x, x_dtype, m, k, ldx, nullptr, eps, qs, n, scale, sdt, bias, true, act, ldact, st);
+    if (rc != 1) return rc;
+  }
   if (wide_pair && m > 16) {
     const void* xin = x;
     int64_t ldin = ldx, left = avail;
