@@ -1,0 +1,51 @@
+"""The dispatch rules that are plain host headers (csrc/*_rule.h), compiled alone and read here on the CPU."""
+
+from __future__ import annotations
+
+import os
+import shutil
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+CSRC = os.path.join(ROOT, "tts-inference_amd", "csrc")
+
+
+def _run(tmp_path, source: str) -> list[list[int]]:
+    """The rows of whole numbers that a program on these headers prints."""
+    cxx = shutil.which("g++") or shutil.which("clang++")
+    if not cxx:
+        pytest.skip("no C++ compiler")
+    src, exe = tmp_path / "rule.cpp", tmp_path / "rule"
+    src.write_text(source)
+    subprocess.run([cxx, "-std=c++17", "-O1", "-Wall", "-Werror", "-I", CSRC, str(src), "-o", str(exe)], check=True)
+    out = subprocess.run([str(exe)], check=True, capture_output=True, text=True).stdout
+    return [[int(v) for v in line.split()] for line in out.splitlines()]
+
+
+def test_rms_norm_rows_of_every_size_take_a_vector_kernel(tmp_path):
+    """16-bit aligned rows: in registers where they fit, in vectors past that (never element by element); the others not."""
+    rows = _run(tmp_path, """
+#include <stdio.h>
+#include "norm_rule.h"
+int main() {
+  const long long ks[] = {8, 512, 520, 1024, 1032, 2048, 2056, 4096, 4104, 8192, 8200, 16384, 1 << 20};
+  const long long ms[] = {1, 1003, 1 << 22, (1 << 22) + 1, 1 << 25};
+  for (long long k : ks)
+    for (long long m : ms)
+      for (int vec = 0; vec < 2; ++vec) {
+        const qtts::NormForm f = qtts::norm_form(vec, m, k);
+        printf("%lld %lld %d %d %d\\n", m, k, vec, f.threads, f.vectors);
+      }
+}
+""")
+    assert len(rows) == 13 * 5 * 2
+    for m, k, vec, threads, vectors in rows:
+        if not vec:
+            assert threads == 0, (m, k)
+        elif k <= 8192 and m <= 1 << 22:
+            assert threads * vectors * 8 >= k and threads * m < 1 << 32, (m, k)
+            assert threads in (64, 128, 256) and (vectors == 1 or threads == 256), (m, k)
+        else:
+            assert (threads, vectors) == (64, 0), (m, k)

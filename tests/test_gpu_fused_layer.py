@@ -103,6 +103,19 @@ def test_rms_norm_row_lengths(ops, dtype, k):
     assert int((err > 0).sum()) <= max(1, y.numel() // 100)
 
 
+@pytest.mark.parametrize("m,k", [(3, 8200), (5, 16384), (2, 65536), ((1 << 22) + 3, 8)])
+def test_rms_norm_past_the_register_kernel(ops, m, k):
+    """Longer rows and more of them than the register kernel takes: within one unit of the value in 64 bits."""
+    g = torch.Generator(device="cuda").manual_seed(k)
+    x = (torch.randn(m, k, device="cuda", generator=g) * 2).to(torch.bfloat16)
+    w = (1 + 0.2 * torch.randn(k, device="cuda", generator=g)).to(torch.bfloat16)
+    y = ops.rms_norm(x, w, 1e-6)
+    for rows in (slice(0, 4096), slice(max(0, m - 4096), m)):
+        xd = x[rows].double()
+        want = (xd * torch.rsqrt(xd.square().mean(1, keepdim=True) + 1e-6) * w.double()).cpu().numpy()
+        assert (np.abs(y[rows].double().cpu().numpy() - want) <= _ulp(want, torch.bfloat16)).all()
+
+
 def test_rms_norm_golden(ops):
     z = np.load(os.path.join(GOLDEN, "rms_norm.npz"))
     eps = float(z["eps"])

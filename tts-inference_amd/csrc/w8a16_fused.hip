@@ -25,6 +25,7 @@
 //    staged rows (9-16 in two row parts of 8, one split).  A fused and a separate RMSNorm
 //    sum in different orders: the fused
 //    result is within the GEMM tolerance of the separate one, not bit-identical.
+#include "norm_rule.h"
 #include "skinny_fused.h"
 #include "wide_rule.h"
 
@@ -107,9 +108,43 @@ __global__ __launch_bounds__(T) void rms_norm_vec_kernel(const XT* __restrict__ 
     }
 }
 
-// The other rows (fp32, ragged or unaligned, longer): one wave a row, 4 rows a workgroup, the row read
-// twice (the second time from cache).
+// The other rows: one wave a row, 4 rows a workgroup, the row read twice (the second time from cache); in vectors where it is
+// 16-bit and aligned (longer rows, or more of them, than the kernel above takes), else element by element.
 constexpr int kNormRowsPerBlock = 4;
+
+template <typename XT>
+__global__ __launch_bounds__(64 * kNormRowsPerBlock) void rms_norm_long_kernel(const XT* __restrict__ x, int64_t ldx,
+                                                                              const XT* __restrict__ w, int k, float eps,
+                                                                              XT* __restrict__ y, int64_t ldy, int m) {
+  const int lane = threadIdx.x & 63;
+  const int64_t row = (int64_t)blockIdx.x * kNormRowsPerBlock + (threadIdx.x >> 6);
+  if (row >= m) return;
+  const XT* xr = x + row * ldx;
+  float ss = 0.0f;
+  for (int e0 = 8 * lane; e0 < k; e0 += 512) {
+    const i32x4_t v = *(const i32x4_t*)(xr + e0);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float a = to_f32(XT{(uint16_t)v[i]}), b = to_f32(XT{(uint16_t)((uint32_t)v[i] >> 16)});
+      ss = __builtin_fmaf(a, a, ss);
+      ss = __builtin_fmaf(b, b, ss);
+    }
+  }
+  ss = wave_sum(ss);
+  const float inv = 1.0f / __builtin_sqrtf(ss / (float)k + eps);
+  for (int e0 = 8 * lane; e0 < k; e0 += 512) {
+    const i32x4_t v = *(const i32x4_t*)(xr + e0), wv = *(const i32x4_t*)(w + e0);
+    i32x4_t o;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const uint32_t p = (uint32_t)v[i], q = (uint32_t)wv[i];
+      const float h0 = (to_f32(XT{(uint16_t)p}) * inv) * to_f32(XT{(uint16_t)q});
+      const float h1 = (to_f32(XT{(uint16_t)(p >> 16)}) * inv) * to_f32(XT{(uint16_t)(q >> 16)});
+      o[i] = (int)pack2_f32<XT>(h0, h1);
+    }
+    *(i32x4_t*)(y + row * ldy + e0) = o;
+  }
+}
 
 template <typename XT>
 __global__ __launch_bounds__(64 * kNormRowsPerBlock) void rms_norm_kernel(const XT* __restrict__ x, int64_t ldx,
@@ -199,21 +234,20 @@ int qtts_launch_silu_mul(const void* gu, int x_dtype, int64_t m, int64_t k, int6
 
 int qtts_launch_rms_norm(const void* x, int x_dtype, int64_t m, int64_t k, int64_t ldx, const void* w, float eps,
                          void* y, int64_t ldy, hipStream_t st) {
-  const int64_t nv = k / 8;
-  const bool vec = x_dtype != QTTS_F32 && k % 8 == 0 && k > 0 && nv <= 1024 && m <= (1 << 22) && (uintptr_t)x % 16 == 0 &&
-                   (uintptr_t)w % 16 == 0 && (uintptr_t)y % 16 == 0 && ldx % 8 == 0 && ldy % 8 == 0;
-  if (vec) {
-    // the fewest threads (64 to 256) that hold the row in one vector each, then more vectors a thread
+  const bool vec = x_dtype != QTTS_F32 && k % 8 == 0 && (uintptr_t)x % 16 == 0 && (uintptr_t)w % 16 == 0 &&
+                   (uintptr_t)y % 16 == 0 && ldx % 8 == 0 && ldy % 8 == 0;
+  const NormForm f = norm_form(vec, m, k);
+  if (f.vectors > 0) {
 #define QTTS_NORM_VEC(T, TH, V)                                                                             \
   qtts::launch(&rms_norm_vec_kernel<T, TH, V>, dim3((unsigned)m), dim3(TH), 0, st, (const T*)x, ldx, (const T*)w, \
                (int)k, eps, (T*)y, ldy)
-#define QTTS_NORM_T(T)                             \
-  do {                                             \
-    if (nv <= 64) QTTS_NORM_VEC(T, 64, 1);         \
-    else if (nv <= 128) QTTS_NORM_VEC(T, 128, 1);  \
-    else if (nv <= 256) QTTS_NORM_VEC(T, 256, 1);  \
-    else if (nv <= 512) QTTS_NORM_VEC(T, 256, 2);  \
-    else QTTS_NORM_VEC(T, 256, 4);                 \
+#define QTTS_NORM_T(T)                                             \
+  do {                                                             \
+    if (f.threads == 64) QTTS_NORM_VEC(T, 64, 1);                  \
+    else if (f.threads == 128) QTTS_NORM_VEC(T, 128, 1);           \
+    else if (f.vectors == 1) QTTS_NORM_VEC(T, 256, 1);             \
+    else if (f.vectors == 2) QTTS_NORM_VEC(T, 256, 2);             \
+    else QTTS_NORM_VEC(T, 256, 4);                                 \
   } while (0)
     if (x_dtype == QTTS_BF16) QTTS_NORM_T(bf16_t);
     else QTTS_NORM_T(f16_t);
@@ -224,7 +258,9 @@ int qtts_launch_rms_norm(const void* x, int x_dtype, int64_t m, int64_t k, int64
   const dim3 grid((unsigned)((m + kNormRowsPerBlock - 1) / kNormRowsPerBlock)), block(64 * kNormRowsPerBlock);
 #define QTTS_NORM(KER, T) \
   qtts::launch(&KER<T>, grid, block, 0, st, (const T*)x, ldx, (const T*)w, (int)k, eps, (T*)y, ldy, (int)m)
-  if (x_dtype == QTTS_BF16) QTTS_NORM(rms_norm_kernel, bf16_t);
+  if (f.threads > 0 && x_dtype == QTTS_BF16) QTTS_NORM(rms_norm_long_kernel, bf16_t);
+  else if (f.threads > 0) QTTS_NORM(rms_norm_long_kernel, f16_t);
+  else if (x_dtype == QTTS_BF16) QTTS_NORM(rms_norm_kernel, bf16_t);
   else if (x_dtype == QTTS_F16) QTTS_NORM(rms_norm_kernel, f16_t);
   else QTTS_NORM(rms_norm_kernel, float);
 #undef QTTS_NORM
