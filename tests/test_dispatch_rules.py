@@ -49,3 +49,28 @@ int main() {
             assert threads in (64, 128, 256) and (vectors == 1 or threads == 256), (m, k)
         else:
             assert (threads, vectors) == (64, 0), (m, k)
+
+
+def test_wide_tiles_are_built_in_the_forms_that_the_rule_chooses(tmp_path):
+    """The launcher builds each tile in the forms its line names, and the rule takes tiles from those lines alone: every line's
+    forms are the ones that some call chooses it in, no more (a kernel nothing reaches) and no fewer."""
+    rows = _run(tmp_path, """
+#include <stdio.h>
+#include "wide_rule.h"
+using namespace qtts;
+int main() {
+  int chosen[kWideTileCount] = {0};
+  for (int k = 64; k <= 6400; k += 64)
+    for (int n = 32; n <= 20000; n += 32)
+      for (int m = 1; m <= 140; ++m)
+        for (int form = 1; form <= 16; form *= 2) {
+          const bool pair = form == kWidePair || form == kWideNormPair, plain = form == kWidePlain || form == kWideFp8;
+          if (pair && n % 32) continue;
+          if (plain && half_cfg(m, n, k).waves) continue;  // the half strips come first
+          const int t = wide_cfg(m, n, k, form);
+          if (t >= 0) chosen[t] |= form;
+        }
+  for (int i = 0; i < kWideTileCount; ++i) printf("%d %d\\n", kWideTiles[i].forms, chosen[i]);
+}
+""")
+    assert rows and all(built == chosen for built, chosen in rows), rows

@@ -25,6 +25,7 @@
 
 #include <algorithm>
 #include <type_traits>
+#include <utility>
 
 #include "common.h"
 #include "layout.h"
@@ -337,49 +338,29 @@ struct WideArgs {
   const void* aux; float eps; const void* res; int64_t ldr; void* y; int64_t ldy; hipStream_t st;
 };
 
-// One launch of a configuration of wide_cfg (wide_rule.h); false when it is not built.
-template <typename XT, int EPI, bool NORM, bool F8W> inline bool launch_wide(const WideCfg& c, const WideArgs& a) {
-  const int64_t strips = (a.n + 15) / 16;
-  const dim3 grid((unsigned)(((strips + c.nb - 1) / c.nb + 7) / 8 * 8), 1, (unsigned)((a.m + 16 * c.mb - 1) / (16 * c.mb)));
-#define QTTS_WIDE(MB, NB, W, CPW, CL)                                                                                \
-  if (c.mb == MB && c.nb == NB && c.waves == W && c.cpw == CPW) {                                                    \
-    qtts::launch_by_policy<std::is_same<XT, bf16_t>::value>([&](auto nt) {                                           \
-      qtts::launch(&w8a16_wide_kernel<XT, MB, NB, W, CPW, CL, EPI, NORM, F8W, decltype(nt)::value>, grid,            \
-                   dim3(W * 64), 0, a.st, a.qs, (const XT*)a.x, a.scale, (const XT*)a.bias, (const XT*)a.aux,        \
-                   (int)a.ldx, (int)a.m, (int)a.n, a.sdt, a.eps, (XT*)a.y, a.ldy, (const XT*)a.res, a.ldr);          \
-    });                                                                                                              \
-    return true;                                                                                                     \
+// One launch of tile I of kWideTiles (wide_rule.h) in its form.
+template <typename XT, int EPI, bool NORM, bool F8W, int FORM, int I> inline void launch_wide_tile(const WideArgs& a) {
+  if constexpr ((kWideTiles[I].forms & FORM) != 0) {
+    constexpr WideTile t = kWideTiles[I];
+    const int64_t strips = (a.n + 15) / 16;
+    const dim3 grid((unsigned)(((strips + t.nb - 1) / t.nb + 7) / 8 * 8), 1, (unsigned)((a.m + 16 * t.mb - 1) / (16 * t.mb)));
+    qtts::launch_by_policy<std::is_same<XT, bf16_t>::value>([&](auto nt) {
+      qtts::launch(&w8a16_wide_kernel<XT, t.mb, t.nb, t.waves, t.cpw, t.cl, EPI, NORM, F8W, decltype(nt)::value>, grid,
+                   dim3(t.waves * 64), 0, a.st, a.qs, (const XT*)a.x, a.scale, (const XT*)a.bias, (const XT*)a.aux,
+                   (int)a.ldx, (int)a.m, (int)a.n, a.sdt, a.eps, (XT*)a.y, a.ldy, (const XT*)a.res, a.ldr);
+    });
   }
-  QTTS_WIDE(1, 1, 8, 2, 2)
-  QTTS_WIDE(1, 2, 8, 2, 2)
-  QTTS_WIDE(1, 3, 8, 2, 2)
-  QTTS_WIDE(1, 4, 8, 2, 2)
-  QTTS_WIDE(2, 2, 8, 2, 2)
-  QTTS_WIDE(2, 3, 8, 2, 2)
-  QTTS_WIDE(2, 4, 8, 2, 2)
-  if constexpr (!NORM) {
-    QTTS_WIDE(4, 3, 8, 2, 2)
-  }
-  QTTS_WIDE(1, 1, 16, 2, 2)
-  QTTS_WIDE(1, 2, 16, 2, 2)
-  QTTS_WIDE(1, 3, 16, 2, 2)
-  QTTS_WIDE(1, 4, 16, 2, 2)
-  if constexpr (!NORM) {
-    QTTS_WIDE(2, 2, 16, 2, 2)
-    QTTS_WIDE(2, 3, 16, 2, 2)
-    QTTS_WIDE(2, 4, 16, 2, 2)
-  }
-  QTTS_WIDE(1, 1, 8, 4, 4)
-  QTTS_WIDE(1, 2, 8, 4, 4)
-  if constexpr (!NORM) {
-    QTTS_WIDE(2, 2, 8, 4, 4)
-    QTTS_WIDE(1, 1, 8, 6, 6)
-    QTTS_WIDE(1, 2, 8, 6, 6)
-    QTTS_WIDE(1, 1, 16, 6, 4)
-    QTTS_WIDE(1, 2, 16, 6, 4)
-  }
-#undef QTTS_WIDE
-  return false;
+}
+
+template <typename XT, int EPI, bool NORM, bool F8W, int... I>
+inline void launch_wide(int tile, const WideArgs& a, std::integer_sequence<int, I...>) {
+  constexpr int form = F8W ? kWideFp8 : (EPI == kEpiPair ? (NORM ? kWideNormPair : kWidePair) : (NORM ? kWideNorm : kWidePlain));
+  (void)((I == tile && (launch_wide_tile<XT, EPI, NORM, F8W, form, I>(a), true)) || ...);
+}
+
+// tile: what wide_cfg gives for the form.
+template <typename XT, int EPI, bool NORM, bool F8W> inline void launch_wide(int tile, const WideArgs& a) {
+  launch_wide<XT, EPI, NORM, F8W>(tile, a, std::make_integer_sequence<int, kWideTileCount>{});
 }
 
 // One launch of a configuration of half_cfg (wide_rule.h).

@@ -8,15 +8,17 @@ using namespace qtts;
 int qtts_launch_w8a16_wide_fused(const void* x, int x_dtype, int64_t m, int64_t k, int64_t ldx, const void* nw, float eps,
                                  const int8_t* qs, int64_t n, const void* scale, int sdt, const void* bias, bool pair,
                                  void* y, int64_t ldy, hipStream_t st) {
-  const WideCfg c = wide_cfg(m, n, k, nw != nullptr, pair);
-  if (c.mb == 0 || ldx > INT32_MAX) return 1;
+  const int tile = wide_cfg(m, n, k, pair ? (nw ? kWideNormPair : kWidePair) : kWideNorm);
+  if (tile < 0 || ldx > INT32_MAX) return 1;
   const WideArgs a{x, m, ldx, qs, n, scale, sdt, bias, nw, eps, nullptr, 0, y, ldy, st};
-  bool ok;
-  if (x_dtype == QTTS_BF16)
-    ok = !pair ? launch_wide<bf16_t, kEpiNone, true, false>(c, a)
-               : (nw ? launch_wide<bf16_t, kEpiPair, true, false>(c, a) : launch_wide<bf16_t, kEpiPair, false, false>(c, a));
-  else
-    ok = !pair ? launch_wide<f16_t, kEpiNone, true, false>(c, a)
-               : (nw ? launch_wide<f16_t, kEpiPair, true, false>(c, a) : launch_wide<f16_t, kEpiPair, false, false>(c, a));
-  return ok ? qtts_check_launch("w8a16_wide_fused") : 1;
+  if (x_dtype == QTTS_BF16) {
+    if (!pair) launch_wide<bf16_t, kEpiNone, true, false>(tile, a);
+    else if (nw) launch_wide<bf16_t, kEpiPair, true, false>(tile, a);
+    else launch_wide<bf16_t, kEpiPair, false, false>(tile, a);
+  } else {
+    if (!pair) launch_wide<f16_t, kEpiNone, true, false>(tile, a);
+    else if (nw) launch_wide<f16_t, kEpiPair, true, false>(tile, a);
+    else launch_wide<f16_t, kEpiPair, false, false>(tile, a);
+  }
+  return qtts_check_launch("w8a16_wide_fused");
 }

@@ -5,9 +5,24 @@
 
 namespace qtts {
 
-struct WideCfg { int mb, nb, waves, cpw; };  // mb == 0: not this kernel
+// The forms of a call: kWidePlain with and without the residual, kWideFp8 the plain form on e4m3 codes.
+enum : int { kWidePlain = 1, kWideNorm = 2, kWidePair = 4, kWideNormPair = 8, kWideFp8 = 16 };
 
-// The automatic choice for an [m, k] x [n, k] call, strip weights: 9 to 128 rows (8 and fewer stay with the
+// A workgroup of `waves` waves, up to cpw chunks (64 columns) of K each, cl of them through LDS; 16 mb rows, nb strips;
+// forms: those that it is built for, the ones that wide_cfg chooses it in.
+struct WideTile { int mb, nb, waves, cpw, cl, forms; };
+
+constexpr WideTile kWideTiles[] = {
+    {1, 1, 8, 2, 2, 31}, {1, 2, 8, 2, 2, 31}, {1, 3, 8, 2, 2, 31}, {1, 4, 8, 2, 2, 31}, {2, 2, 8, 2, 2, 14},
+    {2, 3, 8, 2, 2, 31}, {2, 4, 8, 2, 2, 31}, {4, 3, 8, 2, 2, 4},
+    {1, 1, 16, 2, 2, 31}, {1, 2, 16, 2, 2, 31}, {1, 3, 16, 2, 2, 31}, {1, 4, 16, 2, 2, 31}, {2, 2, 16, 2, 2, 21},
+    {2, 3, 16, 2, 2, 21}, {2, 4, 16, 2, 2, 21},
+    {1, 1, 8, 4, 4, 31}, {1, 2, 8, 4, 4, 31}, {2, 2, 8, 4, 4, 21},
+    {1, 1, 8, 6, 6, 21}, {1, 2, 8, 6, 6, 21},
+    {1, 1, 16, 6, 4, 21}, {1, 2, 16, 6, 4, 21}};
+constexpr int kWideTileCount = (int)(sizeof(kWideTiles) / sizeof(kWideTiles[0]));
+
+// The tile of kWideTiles for the automatic choice of an [m, k] x [n, k] call on strip weights, or -1: 9 to 128 rows (8 and fewer stay with the
 // decode kernel, whose half strips and row staging are faster there; with the norm inside and K <= 1024 from 5
 // rows: 8 rows of the predictor's qkv 5.50 -> 5.00 us, of its gate_up with the activation 6.59 -> 5.65) where K is a built
 // product of waves and chunks and one of the built tiles covers the call in a single round of
@@ -22,37 +37,30 @@ struct WideCfg { int mb, nb, waves, cpw; };  // mb == 0: not this kernel
 // pair: a gate_up weight with its activation.  K = 1024 past 48 rows: plain and residual calls stay with the
 // tile kernel, whose result the automatic choice is held to bit for bit there (they would
 // gain 0.1-0.9 us a call).
-inline WideCfg wide_cfg(int64_t m, int64_t n, int64_t k, bool norm = false, bool pair = false) {
-  WideCfg best{0, 0, 0, 0};
-  if (k == 1024 && m > 48 && !norm && !pair) return best;
-  if (m < (norm && k <= 1024 ? 5 : 9) || m > 128 || n <= 0 || n > (1 << 30)) return best;
+inline int wide_cfg(int64_t m, int64_t n, int64_t k, int form) {
+  const bool norm = (form & (kWideNorm | kWideNormPair)) != 0, pair = (form & (kWidePair | kWideNormPair)) != 0;
+  if (k == 1024 && m > 48 && !norm && !pair) return -1;
+  if (m < (norm && k <= 1024 ? 5 : 9) || m > 128 || n <= 0 || n > (1 << 30)) return -1;
   const int64_t strips = (n + 15) / 16;
-  struct Tile { int mb, nb; };
-  static const Tile t82[] = {{1, 1}, {1, 2}, {1, 3}, {1, 4}, {2, 2}, {2, 3}, {2, 4}, {4, 3}};
-  static const Tile t162[] = {{1, 1}, {1, 2}, {1, 3}, {1, 4}, {2, 2}, {2, 3}, {2, 4}};
-  static const Tile t84[] = {{1, 1}, {1, 2}, {2, 2}};
-  static const Tile t86[] = {{1, 1}, {1, 2}};
-  const Tile* tiles;
-  int count, w, c;
+  int waves, cpw;
   switch (k) {
-    case 1024: tiles = t82, count = 8, w = 8, c = 2; break;
-    case 2048:
-      if (strips > 128) tiles = t162, count = 7, w = 16, c = 2;
-      else tiles = t84, count = 3, w = 8, c = 4;
-      break;
-    case 3072: tiles = t86, count = 2, w = 8, c = 6; break;
-    case 6144: tiles = t86, count = 2, w = 16, c = 6; break;
-    default: return best;
+    case 1024: waves = 8, cpw = 2; break;
+    case 2048: waves = strips > 128 ? 16 : 8, cpw = strips > 128 ? 2 : 4; break;
+    case 3072: waves = 8, cpw = 6; break;
+    case 6144: waves = 16, cpw = 6; break;
+    default: return -1;
   }
+  int best = -1;
   int64_t best_cost = 0;
-  for (int i = 0; i < count; ++i) {
-    const int mb = tiles[i].mb, nb = tiles[i].nb;
-    if (16 * mb >= m + 16) continue;  // a row block with no row of the call
-    if ((strips + nb - 1) / nb * ((m + 16 * mb - 1) / (16 * mb)) > 256) continue;
-    if (norm && (16 * mb * k > 32768 || k > 2048)) continue;
-    const int64_t cost = norm ? 8 * mb + nb : 2 * mb + nb;  // bytes a workgroup over 16 K
-    if (best.mb == 0 || cost < best_cost) {
-      best = WideCfg{mb, nb, w, c};
+  for (int i = 0; i < kWideTileCount; ++i) {
+    const WideTile& t = kWideTiles[i];
+    if (t.waves != waves || t.cpw != cpw || !(t.forms & form)) continue;
+    if (16 * t.mb >= m + 16) continue;  // a row block with no row of the call
+    if ((strips + t.nb - 1) / t.nb * ((m + 16 * t.mb - 1) / (16 * t.mb)) > 256) continue;
+    if (norm && (16 * t.mb * k > 32768 || k > 2048)) continue;
+    const int64_t cost = norm ? 8 * t.mb + t.nb : 2 * t.mb + t.nb;  // bytes a workgroup over 16 K
+    if (best < 0 || cost < best_cost) {
+      best = i;
       best_cost = cost;
     }
   }
@@ -76,7 +84,7 @@ inline HalfCfg half_cfg(int64_t m, int64_t n, int64_t k) {
 
 // Whether the automatic choice runs a plain (or residual) call on the wide kernels.
 inline bool wide_takes(int64_t m, int64_t n, int64_t k) {
-  return half_cfg(m, n, k).waves > 0 || wide_cfg(m, n, k).mb > 0;
+  return half_cfg(m, n, k).waves > 0 || wide_cfg(m, n, k, kWidePlain) >= 0;
 }
 
 }  // namespace qtts
