@@ -74,3 +74,30 @@ int main() {
 }
 """)
     assert rows and all(built == chosen for built, chosen in rows), rows
+
+
+def test_decode_row_parts_keep_9_to_16_rows_of_few_strips(tmp_path):
+    """65 to 128 strips at 9-16 rows, where two row parts of the decode kernel fill the GPU and the wide kernel does not: the
+    K at which they measured faster stay there, and the lines lie at 16 rows and 64 / 128 strips."""
+    rows = _run(tmp_path, """
+#include <stdio.h>
+#include "wide_rule.h"
+using namespace qtts;
+int main() {
+  const int ks[] = {1024, 2048, 3072, 6144}, ns[] = {1024, 1056, 2048, 2080}, ms[] = {9, 12, 16, 17};
+  for (int k : ks)
+    for (int n : ns)
+      for (int m : ms)
+        for (int form = 1; form <= 16; form *= 2) printf("%d %d %d %d %d\\n", k, n, m, form, wide_cfg(m, n, k, form));
+}
+""")
+    taken = {tuple(r[:4]): r[4] >= 0 for r in rows}
+    plain, norm, pair, norm_pair, fp8 = 1, 2, 4, 8, 16
+    for n in (1056, 2048):
+        for m in (9, 12, 16):
+            for form in (plain, fp8):
+                assert not taken[6144, n, m, form] and not taken[2048, n, m, form]
+                assert taken[1024, n, m, form] and taken[3072, n, m, form] and taken[6144, n, 17, form]
+            assert not taken[2048, n, m, norm] and not taken[2048, n, m, pair]
+            assert taken[2048, n, m, norm_pair] and taken[6144, n, m, pair] and taken[2048, n, 17, norm]
+    assert all(taken[k, 2080, m, plain] for k in (2048, 6144) for m in (9, 16))

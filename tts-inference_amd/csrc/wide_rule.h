@@ -22,6 +22,16 @@ constexpr WideTile kWideTiles[] = {
     {1, 1, 16, 6, 4, 21}, {1, 2, 16, 6, 4, 21}};
 constexpr int kWideTileCount = (int)(sizeof(kWideTiles) / sizeof(kWideTiles[0]));
 
+// Whether the decode kernel's row parts (skinny.h) keep a call of 9 to 16 rows: on 65 to 128 strips their two parts make 256
+// workgroups of 8 staged rows, against this kernel's 128 at most.  Measured at N = 1040 .. 2048, us a call, decode kernel -> wide:
+// K = 6144 plain at 12 / 16 rows 5.64 / 5.60 -> 6.08 / 6.40, residual 6.17 / 6.19 -> 6.67 / 7.06; K = 2048 with the norm 4.81 -> 5.38,
+// with the activation 3.56 -> 3.86, residual 3.63 -> 3.88, plain the same; K = 1024 and 3072 0.2 to 0.6 faster, and
+// the norm with the activation 0.6 to 1.6 everywhere.  (The activation alone at K = 6144 has no decode form: 0.9 to 1.4 faster.)
+inline bool row_parts_keep(int64_t m, int64_t strips, int64_t k, int form) {
+  if (m > 16 || strips <= 64 || strips > 128 || form == kWideNormPair || (form == kWidePair && k > 4096)) return false;
+  return k > 3072 || (k > 1024 && k <= 2048);
+}
+
 // The tile of kWideTiles for the automatic choice of an [m, k] x [n, k] call on strip weights, or -1: 9 to 128 rows (8 and fewer stay with the
 // decode kernel, whose half strips and row staging are faster there; with the norm inside and K <= 1024 from 5
 // rows: 8 rows of the predictor's qkv 5.50 -> 5.00 us, of its gate_up with the activation 6.59 -> 5.65) where K is a built
@@ -42,6 +52,7 @@ inline int wide_cfg(int64_t m, int64_t n, int64_t k, int form) {
   if (k == 1024 && m > 48 && !norm && !pair) return -1;
   if (m < (norm && k <= 1024 ? 5 : 9) || m > 128 || n <= 0 || n > (1 << 30)) return -1;
   const int64_t strips = (n + 15) / 16;
+  if (row_parts_keep(m, strips, k, form)) return -1;
   int waves, cpw;
   switch (k) {
     case 1024: waves = 8, cpw = 2; break;
