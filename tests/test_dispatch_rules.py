@@ -101,3 +101,26 @@ int main() {
             assert not taken[2048, n, m, norm] and not taken[2048, n, m, pair]
             assert taken[2048, n, m, norm_pair] and taken[6144, n, m, pair] and taken[2048, n, 17, norm]
     assert all(taken[k, 2080, m, plain] for k in (2048, 6144) for m in (9, 16))
+
+
+def test_wide_rule_takes_every_k_that_a_built_run_holds(tmp_path):
+    """No list of K: each multiple of 64 in the range takes tiles whose waves hold it in the shortest built runs, each multiple of
+    128 the half strips; the ends of the range."""
+    rows = _run(tmp_path, """
+#include <stdio.h>
+#include "wide_rule.h"
+using namespace qtts;
+int main() {
+  for (int k = 1; k <= 8192; ++k) {
+    const int t = wide_cfg(27, 2048, k, kWidePlain);
+    const HalfCfg h = half_cfg(8, 2048, k);
+    printf("%d %d %d %d\\n", k, t < 0 ? 0 : kWideTiles[t].waves, t < 0 ? 0 : kWideTiles[t].cpw, h.waves * h.upw);
+  }
+}
+""")
+    for k, waves, cpw, units in rows:
+        assert (waves > 0) == (k % 64 == 0 and 512 < k <= 6144), k
+        if waves:
+            assert waves <= k // 64 <= waves * cpw and (k // 64 > 3 * 16 or waves * cpw <= 48), k
+        assert (units > 0) == (k % 128 == 0 and 512 < k <= 6144), k
+        assert not units or k // 128 <= units, k

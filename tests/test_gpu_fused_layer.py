@@ -340,6 +340,10 @@ WIDE = [(5, 4096, 1024), (9, 4096, 1024), (16, 100, 1024), (17, 6144, 1024), (33
         (65, 6144, 1024), (96, 6144, 1024), (128, 6144, 1024), (9, 12288, 2048), (31, 12288, 2048), (47, 4096, 2048),
         (128, 4096, 2048), (27, 2048, 2048), (127, 2048, 2048), (12, 1000, 3072), (97, 1024, 3072), (13, 2048, 6144),
         (32, 2048, 6144), (64, 2048, 6144)]
+# K between the tiles' full runs: waves whose runs differ by one chunk, each group of tiles at the ends of its range of K
+WIDE_K = [(5, 4096, 640), (9, 1040, 576), (16, 4096, 960), (48, 1000, 704), (17, 6144, 1088), (33, 2048, 1088), (64, 1040, 1984),
+          (128, 4096, 1984), (9, 4096, 2112), (27, 1000, 2624), (97, 1024, 3008), (12, 4096, 3136), (32, 2048, 5120), (64, 2048, 6080),
+          (27, 12288, 1536)]
 
 
 def _ref64(h, q, s, b):
@@ -362,7 +366,7 @@ def _bar_product(y, gate, up, what):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("m,n,k", WIDE)
+@pytest.mark.parametrize("m,n,k", WIDE + WIDE_K)
 def test_wide_calls(ops, m, n, k, dtype):
     """The automatic choice at 9-128 rows (the one-round tiles): every form against float64, the
     residual bit for bit the plain call's, strided rows, and rows that do not meet (a row of infinities and
@@ -391,7 +395,7 @@ def test_wide_calls(ops, m, n, k, dtype):
             _bar_product(act.double().cpu().numpy(), full[:, : n // 2], full[:, n // 2:], what + str(list(kw)))
 
 
-@pytest.mark.parametrize("m,n,k", [(9, 4096, 1024), (33, 6144, 1024), (47, 4096, 2048), (97, 1024, 3072), (64, 2048, 6144)])
+@pytest.mark.parametrize("m,n,k", [(9, 4096, 1024), (33, 6144, 1024), (47, 4096, 2048), (97, 1024, 3072), (64, 2048, 6144)] + WIDE_K)
 def test_wide_fp8_codes(ops, m, n, k):
     """The same kernel on e4m3 codes: against float64."""
     g = torch.Generator(device="cuda").manual_seed(m + n)
@@ -399,3 +403,30 @@ def test_wide_fp8_codes(ops, m, n, k):
     q, s = ops.pack_fp8(w)
     x = torch.randn(m, k, device="cuda", generator=g).to(torch.bfloat16)
     assert_close(ops.fp8w_gemm_strips(x, ops.fp8w_strips(q), n, s), _ref64(x, q.float(), s, None), f"wide fp8 {m} {n} {k}")
+
+
+# (m, n, k) of the half strips: idle waves (K / 128 below the waves), runs that differ by one, whole ones; ragged rows and columns
+HALF = [(5, 200, 640), (8, 2048, 768), (7, 1000, 1152), (16, 1024, 1920), (8, 2040, 2048), (12, 1000, 2176), (16, 1024, 3072),
+        (13, 1000, 5120), (8, 2048, 6016), (5, 2048, 6144)]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("m,n,k", HALF)
+def test_wide_half_strips(ops, m, n, k, dtype):
+    """The half strips' automatic calls: against float64 on int8 and e4m3 codes, the residual bit for bit the plain call's, and
+    rows that do not meet."""
+    q, s, qs = _weights(ops, n, k, dtype, 6)
+    g = torch.Generator(device="cuda").manual_seed(m * 5 + k)
+    x = torch.randn(m, k + 8, device="cuda", generator=g).to(dtype)[:, :k]
+    b = torch.randn(n, device="cuda", generator=g).to(dtype)
+    what = f"half m={m} n={n} k={k} {dtype}"
+    y = ops.w8a16_gemm_strips(x, qs, n, s, b)
+    assert_close(y, _ref64(x, q, s, b), what)
+    res = torch.randn(m, n + 3, device="cuda", generator=g).to(dtype)[:, :n]
+    assert torch.equal(ops.w8a16_fused_gemm_strips(x, qs, n, s, b, residual=res), res + y), what
+    odd = x.clone()
+    odd[0], odd[m // 2] = float("inf"), float("nan")
+    rest = [i for i in range(m) if i not in (0, m // 2)]
+    assert torch.equal(ops.w8a16_gemm_strips(odd, qs, n, s, b)[rest], y[rest]), what
+    qf, sf = ops.pack_fp8((torch.randn(n, k, device="cuda", generator=g) * 0.02).to(dtype))
+    assert_close(ops.fp8w_gemm_strips(x, ops.fp8w_strips(qf), n, sf, b), _ref64(x, qf.float(), sf, b), what + " e4m3")

@@ -1,26 +1,24 @@
-// The W8A16 kernel for 9 to 128 rows of weights that fill the GPU once (decode batches past 8, the code
-// predictor's prefix walk, short prompts): strip weights, K = 64 W CPW.
+// The W8A16 kernels for 5 to 128 rows of weights that fill the GPU once (decode batches, the code predictor's prefix walk, short
+// prompts) on strip weights, and for more rows of very few strips; the rule, row by row, is wide_rule.h.
 //
 // These calls are bound by latency and by the bytes each compute unit pulls through L2, not by the
 // matrix cores: a ring of LDS stages (tile_w8a16.h) spends a wait and a barrier on each of its 8-48
 // stages.  Here a workgroup owns 16 MB rows x 16 NB columns and all of K; its W waves split K into
-// runs of CPW chunks, and a wave issues every load of its run before it consumes any: the activation
+// runs of up to CPW chunks, and a wave issues every load of its run before it consumes any: the activation
 // rows straight to its own LDS block in whole cache lines (16-byte pieces swizzled, as pipe.h's
 // stages), the weights to registers.  A call is one memory round trip and one reduction
 // through LDS.  (Activation operands loaded to registers in MFMA lane order, as the decode kernel's
 // direct form does, touch each line twice at half width: 0.5-1.5 us a call slower at 32 rows.)
 //
-// Measured in graphs over distinct weights (5 layers of the predictor's, 12-28 of the talker's), us a call,
-// the former automatic choice -> this kernel at 16 / 32 / 64 / 128 rows: the talker's qkv 4.83 / 6.89 /
-// 7.40 / 7.94 -> 4.01 / 4.49 / 5.52 / 6.95, o_proj 3.76 / 5.51 / 7.30 / 7.31 -> 3.64 / 3.69 / 4.30 / 5.01,
-// gate_up at 16 / 32 9.58 / 9.76 -> 7.42 / 8.30, down_proj at 32 / 64 9.48 / 9.64 -> 6.68 / 7.73; the
-// predictor's qkv 4.71 / 5.24 / 6.04 / 6.24 -> 4.32 / 4.73 / 5.13 / 6.10, o_proj 4.42 / 4.93 / 5.90 /
-// 7.94 -> 4.39 / 4.48 / 4.66 / 5.39, gate_up 5.50 / 7.18 / 6.35 / 8.11 -> 4.66 / 5.10 / 5.83 / 7.45,
-// down_proj 5.13 / 6.08 / 7.90 / 8.48 -> 4.94 / 5.03 / 5.25 / 5.94.  With the RMSNorm inside against the
-// norm before the GEMM (or the decode kernel's): predictor qkv 6.64 / 7.66 / 8.76 / 9.05 -> 5.06 / 5.50 / 6.14 /
-// 7.55, talker qkv 6.96 / 9.29 / 10.17 -> 5.88 / 6.54 / 7.88 to 64 rows; gate_up with norm and activation 8.24 /
-// 10.16 / 9.60 -> 5.72 / 6.17 / 7.48 (predictor), 13.97 -> 10.03 at 16 rows (talker).  The floor of a call
-// is the 1.6 us launch, one memory round trip and 2-13 MB at 5.1 TB/s.
+// Measured in graphs over distinct weights (5 of the predictor's, 12 of the talker's), us a call, the former automatic choice ->
+// this kernel, at the row counts of 16 / 32 / 64 / 128 that come here: the talker's qkv 4.33 / 6.34 / 7.39 / 7.94 -> 3.82 / 4.28 /
+// 5.44 / 6.74, o_proj from 32 rows 5.20 / 7.37 / 7.32 -> 3.65 / 4.41 / 5.06, gate_up at 16 / 32 9.52 / 10.17 -> 7.04 / 7.96, down_proj at
+// 32 / 64 9.36 / 9.54 -> 6.37 / 7.54; the predictor's qkv and gate_up at 16 / 32 3.21 / 4.10 -> 2.73 / 3.29 and 4.44 / 6.08 -> 3.31 / 3.78, its
+// o_proj from 32 rows 3.72 / 4.80 / 7.06 -> 3.10 / 3.34 / 4.11, down_proj 4.83 / 7.00 / 7.68 -> 3.59 / 3.83 / 4.83.  With the RMSNorm inside
+// against the norm before the GEMM (or the decode kernel's): predictor qkv 5.58 / 6.64 / 7.96 / 8.36 -> 3.72 / 4.14 / 4.87 / 6.42, talker
+// qkv to 64 rows 6.53 / 9.67 / 10.87 -> 5.83 / 6.30 / 7.62; gate_up with norm and activation to 64 rows 7.24 / 10.74 / 10.54 -> 4.46 /
+// 4.92 / 6.35 (predictor), at 16 13.08 -> 9.42 (talker).  The floor of a call is the 1.6 us launch, one memory round trip and 2-13 MB
+// at 5.1 TB/s.
 #pragma once
 
 #include <algorithm>
@@ -47,17 +45,17 @@ __device__ __forceinline__ float add_row_lanes(float v) {
 // EPI: tile_w8a16.h's epilogues.  NORM: the input is RMSNorm(x) with weight aux and epsilon eps,
 // rounded as the reference rounds it (skinny.h: kProRmsNorm): each wave sums x^2 over its run, the
 // waves meet at one fence-free barrier while the weights stay in flight, and each scales its operands.
+// FIT: K = 64 W CPW, every run a constant (the norm with K = 2048 at 32 / 64 rows 6.5 / 7.7 us, 6.8 / 8.3 with the runs computed).
 // CL: chunks of a run that go through LDS; the rest load to registers in lane order (LDS holds no more).
 // NT: the weight policy, as in skinny.h (alone, streaming loads measure 0.1-0.8 us a call slower; in a 12-layer
 // talker step they win, 32 rows 382.0 -> 379.0 us, 8 rows 289.2 -> 280.7 with the half strips below).
-template <typename XT, int MB, int NB, int W, int CPW, int CL, int EPI, bool NORM, bool F8W, bool NT>
+template <typename XT, int MB, int NB, int W, int CPW, int CL, int EPI, bool NORM, bool F8W, bool NT, bool FIT>
 __global__ __launch_bounds__(W * 64) void w8a16_wide_kernel(
     const int8_t* __restrict__ qs, const XT* __restrict__ x, const void* scale, const XT* bias, const XT* aux, int ldx,
-    int M, int N, int sdt, float eps, XT* y, int64_t ldy, const XT* res, int64_t ldr) {
+    int M, int N, int kdt, float eps, XT* y, int64_t ldy, const XT* res, int64_t ldr) {
   typedef mfma16<XT> MM;
   typedef typename MM::vec V;
   constexpr int XI = 2 * MB * CL, P = 8 * CL;  // direct loads a wave, 16-byte pieces a row of its block
-  constexpr int nchunks = W * CPW;
   static_assert(CL <= CPW && (CL % 2 == 0 || CL == 1 || CL == 3), "pieces in groups of 16, or of 8");
   __shared__ __align__(1024) uint8_t lds[W][1024 * (2 * MB * CL > MB * NB ? 2 * MB * CL : MB * NB)];
   __shared__ uint32_t epi_sc[16 * NB], epi_bi[16 * NB];  // scale and bias bits, column by column
@@ -67,29 +65,41 @@ __global__ __launch_bounds__(W * 64) void w8a16_wide_kernel(
   if (s0 >= strips) return;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r = lane & 15, g = lane >> 4;
-  const int wc0 = wave * CPW;
+  const int chunks = FIT ? W * CPW : kdt >> 8, sdt = kdt & 0xff;  // K / 64, the scales' type
+  // The wave's run of K: run chunks from wc0 (0 to CPW; the runs of a call differ by one at most).  A run shorter
+  // than CPW loads its last chunk again in the slots past it, and leaves them out of the sums.
+  const int wc0 = FIT ? wave * CPW : wave * (chunks / W) + min(wave, chunks % W);
+  const int run = FIT ? CPW : chunks / W + (wave < chunks % W ? 1 : 0);
+  const int last = min(max(run, 1), chunks - wc0) - 1;  // of the run, counted from wc0 (-1: a wave of no chunks)
+  auto at = [&](int u) { return FIT ? u : min(u, last); };
 
   // Position of piece p of a row in the wave's block (an involution): conflict-free operand reads.
   auto swz = [](int row, int p) { return CL % 2 == 0 ? p ^ (row & 15) : ((p & ~7) | swizzle8(row, p & 7)); };
+  const XT* xw = x + wc0 * 64;
+  auto load_rows = [&](auto whole) __attribute__((always_inline)) {
 #pragma unroll
-  for (int i = 0; i < XI; ++i) {
-    const int flat = i * 64 + lane, row = flat / P, p = flat % P;
-    load_to_lds16(x + (int64_t)min(y0 + row, M - 1) * ldx + wc0 * 64 + 8 * swz(row, p), &lds[wave][i * 1024]);
-  }
+    for (int i = 0; i < XI; ++i) {
+      const int flat = i * 64 + lane, row = flat / P, p = swz(row, flat % P);
+      const int col = decltype(whole)::value ? 8 * p : at(p >> 3) * 64 + 8 * (p & 7);
+      load_to_lds16(xw + (int64_t)min(y0 + row, M - 1) * ldx + col, &lds[wave][i * 1024]);
+    }
+  };
+  if (FIT || run >= CL) load_rows(std::true_type{});
+  else load_rows(std::false_type{});
   i32x4_t w[CPW][NB], xa[CPW][MB], xb[CPW][MB], nw[NORM ? CPW : 1][2];
 #pragma unroll
   for (int u = CL; u < CPW; ++u)
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb) {
-      const XT* p = x + (int64_t)min(y0 + 16 * mb + r, M - 1) * ldx + (wc0 + u) * 64 + 16 * g;
+      const XT* p = x + (int64_t)min(y0 + 16 * mb + r, M - 1) * ldx + (wc0 + at(u)) * 64 + 16 * g;
       xa[u][mb] = *(const i32x4_t*)p;
       xb[u][mb] = *(const i32x4_t*)(p + 8);
     }
   if constexpr (NORM) {
 #pragma unroll
     for (int u = 0; u < CPW; ++u) {
-      nw[u][0] = *(const i32x4_t*)(aux + (wc0 + u) * 64 + 16 * g);
-      nw[u][1] = *(const i32x4_t*)(aux + (wc0 + u) * 64 + 16 * g + 8);
+      nw[u][0] = *(const i32x4_t*)(aux + (wc0 + at(u)) * 64 + 16 * g);
+      nw[u][1] = *(const i32x4_t*)(aux + (wc0 + at(u)) * 64 + 16 * g + 8);
     }
   }
   __builtin_amdgcn_sched_barrier(0);
@@ -99,12 +109,12 @@ __global__ __launch_bounds__(W * 64) void w8a16_wide_kernel(
     const int8_t* wp;
     if constexpr (EPI == kEpiPair) {  // (N % 32 == 0: both halves sit in whole strips)
       const int R = 8 * s + (r & 7) + (r < 8 ? 0 : (N >> 1));
-      wp = qs + ((int64_t)(R >> 4) * nchunks + wc0) * 1024 + ((R & 15) + 16 * g) * 16;
+      wp = qs + ((int64_t)(R >> 4) * chunks + wc0) * 1024 + ((R & 15) + 16 * g) * 16;
     } else {
-      wp = qs + ((int64_t)s * nchunks + wc0) * 1024 + lane * 16;
+      wp = qs + ((int64_t)s * chunks + wc0) * 1024 + lane * 16;
     }
 #pragma unroll
-    for (int u = 0; u < CPW; ++u) w[u][nb] = load_weight<NT>(wp + u * 1024);
+    for (int u = 0; u < CPW; ++u) w[u][nb] = load_weight<NT>(wp + at(u) * 1024);
   }
   __builtin_amdgcn_sched_barrier(0);
 
@@ -147,9 +157,11 @@ __global__ __launch_bounds__(W * 64) void w8a16_wide_kernel(
     for (int mb = 0; mb < MB; ++mb) {
       float ss = 0.0f;
 #pragma unroll
-      for (int u = 0; u < CPW; ++u)
+      for (int u = 0; u < CPW; ++u) {
+        if (!FIT && u >= run) break;
 #pragma unroll
         for (int i = 0; i < 4; ++i) ss = sq2_acc<XT>((uint32_t)xb[u][mb][i], sq2_acc<XT>((uint32_t)xa[u][mb][i], ss));
+      }
       ss = add_row_lanes(ss);
       if (g == 0) nss[wave][16 * mb + r] = ss;
     }
@@ -160,7 +172,7 @@ __global__ __launch_bounds__(W * 64) void w8a16_wide_kernel(
       float t = 0.0f;
 #pragma unroll
       for (int v = 0; v < W; ++v) t += nss[v][16 * mb + r];
-      const float inv = 1.0f / __builtin_sqrtf(t / (float)(64 * nchunks) + eps);
+      const float inv = 1.0f / __builtin_sqrtf(t / (float)(64 * chunks) + eps);
 #pragma unroll
       for (int u = 0; u < CPW; ++u)
 #pragma unroll
@@ -182,7 +194,8 @@ __global__ __launch_bounds__(W * 64) void w8a16_wide_kernel(
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb) acc[nb][mb] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-  for (int u = 0; u < CPW; ++u)
+  for (int u = 0; u < CPW; ++u) {
+    if (!FIT && u >= run) break;
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) {
       const V wlo = wcvt<F8W, XT>((uint32_t)w[u][nb][0], (uint32_t)w[u][nb][1]);
@@ -192,6 +205,7 @@ __global__ __launch_bounds__(W * 64) void w8a16_wide_kernel(
 #pragma unroll
       for (int mb = 0; mb < MB; ++mb) acc[nb][mb] = MM::mma(whi, __builtin_bit_cast(V, xb[u][mb]), acc[nb][mb]);
     }
+  }
 
   // Each wave's sums over its own rows block (its reads of it are done: the MFMAs above waited for them).
 #pragma unroll
@@ -266,34 +280,45 @@ __global__ __launch_bounds__(W * 64) void w8a16_wide_kernel(
 // The same for up to 8 rows a workgroup on few strips: a workgroup takes half a strip (8 weight rows) of one
 // 8-row part of the call, so 64 or 128 strips still spread over the GPU.  One MFMA covers two chunks ("a unit"), as
 // skinny.h's half strips: A rows 0-7 and B columns 0-7 hold the even chunk, rows 8-15 and columns 8-15 the odd
-// one, and the two diagonal blocks of D are added in the epilogue.  K = 128 W UPW.  What it has over the half strips
+// one, and the two diagonal blocks of D are added in the epilogue.  What it has over the half strips
 // of skinny.h: the rows go straight to LDS (no registers, no LDS writes) and 8-12 waves share a row's loads.
 // Measured as above, us a call, skinny.h's half strips (9-16 rows: the kernel above) -> this one, with the
 // residual add, at 8 / 16 rows: the talker's o_proj 3.51 -> 3.23 at 8, its down_proj 6.11 -> 4.62; the predictor's
 // o_proj 4.37 / 4.60 -> 3.92 / 4.07, its down_proj 5.07 / 5.02 -> 4.14 / 4.35; its 1-stream frame 1243 -> 1158.
-template <typename XT, int W, int UPW, int EPI, bool F8W, bool NT>
+template <typename XT, int W, int UPW, int EPI, bool F8W, bool NT, bool FIT>
 __global__ __launch_bounds__(W * 64) void w8a16_wide_half_kernel(
-    const int8_t* __restrict__ qs, const XT* __restrict__ x, const void* scale, const XT* bias, int ldx, int M, int N, int sdt,
+    const int8_t* __restrict__ qs, const XT* __restrict__ x, const void* scale, const XT* bias, int ldx, int M, int N, int kdt,
     XT* y, int64_t ldy, const XT* res, int64_t ldr) {
   typedef mfma16<XT> MM;
   typedef typename MM::vec V;
-  constexpr int P = 16 * UPW, XI = 2 * UPW, nchunks = 2 * W * UPW;
+  constexpr int P = 16 * UPW, XI = 2 * UPW;
   __shared__ __align__(1024) uint8_t lds[W][XI * 1024];
   const int strip = blockIdx.x >> 1, part = (blockIdx.x & 1) * 8, y0 = blockIdx.z * 8;
   if (strip * 16 + part >= N) return;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r = lane & 15, g = lane >> 4;
-  const int u0 = wave * UPW;
+  const int units = FIT ? W * UPW : kdt >> 8, sdt = kdt & 0xff;  // K / 128, the scales' type
+  // The wave's run of units, as the kernel above's of chunks
+  const int u0 = FIT ? wave * UPW : wave * (units / W) + min(wave, units % W);
+  const int run = FIT ? UPW : units / W + (wave < units % W ? 1 : 0);
+  const int last = min(max(run, 1), units - u0) - 1;
+  auto at = [&](int u) { return FIT ? u : min(u, last); };
+  const XT* xw = x + u0 * 128;
+  auto load_rows = [&](auto whole) __attribute__((always_inline)) {
 #pragma unroll
-  for (int i = 0; i < XI; ++i) {
-    const int flat = i * 64 + lane, row = flat / P, p = flat % P;
-    load_to_lds16(x + (int64_t)min(y0 + row, M - 1) * ldx + u0 * 128 + 8 * (p ^ row), &lds[wave][i * 1024]);
-  }
+    for (int i = 0; i < XI; ++i) {
+      const int flat = i * 64 + lane, row = flat / P, p = flat % P ^ row;
+      const int col = decltype(whole)::value ? 8 * p : at(p >> 4) * 128 + 8 * (p & 15);
+      load_to_lds16(xw + (int64_t)min(y0 + row, M - 1) * ldx + col, &lds[wave][i * 1024]);
+    }
+  };
+  if (FIT || run == UPW) load_rows(std::true_type{});
+  else load_rows(std::false_type{});
   __builtin_amdgcn_sched_barrier(0);
   i32x4_t w[UPW];
-  const int8_t* wp = qs + ((int64_t)strip * nchunks + 2 * u0 + (r >> 3)) * 1024 + (part + (r & 7) + 16 * g) * 16;
+  const int8_t* wp = qs + ((int64_t)strip * 2 * units + 2 * u0 + (r >> 3)) * 1024 + (part + (r & 7) + 16 * g) * 16;
 #pragma unroll
-  for (int u = 0; u < UPW; ++u) w[u] = load_weight<NT>(wp + u * 2048);
+  for (int u = 0; u < UPW; ++u) w[u] = load_weight<NT>(wp + at(u) * 2048);
   __builtin_amdgcn_sched_barrier(0);
   // output (row m, column n) of lane: n = lane % 8, m = lane / 8
   const int on = min(strip * 16 + part + (lane & 7), N - 1), om = min(y0 + (lane >> 3), M - 1);
@@ -313,6 +338,7 @@ __global__ __launch_bounds__(W * 64) void w8a16_wide_half_kernel(
   f32x4_t acc = {0, 0, 0, 0};
 #pragma unroll
   for (int u = 0; u < UPW; ++u) {
+    if (!FIT && u >= run) break;
     acc = MM::mma(wcvt<F8W, XT>((uint32_t)w[u][0], (uint32_t)w[u][1]), xa[u], acc);
     acc = MM::mma(wcvt<F8W, XT>((uint32_t)w[u][2], (uint32_t)w[u][3]), xb[u], acc);
   }
@@ -334,7 +360,7 @@ __global__ __launch_bounds__(W * 64) void w8a16_wide_half_kernel(
 }
 
 struct WideArgs {
-  const void* x; int64_t m, ldx; const int8_t* qs; int64_t n; const void* scale; int sdt; const void* bias;
+  const void* x; int64_t m, k, ldx; const int8_t* qs; int64_t n; const void* scale; int sdt; const void* bias;
   const void* aux; float eps; const void* res; int64_t ldr; void* y; int64_t ldy; hipStream_t st;
 };
 
@@ -344,10 +370,15 @@ template <typename XT, int EPI, bool NORM, bool F8W, int FORM, int I> inline voi
     constexpr WideTile t = kWideTiles[I];
     const int64_t strips = (a.n + 15) / 16;
     const dim3 grid((unsigned)(((strips + t.nb - 1) / t.nb + 7) / 8 * 8), 1, (unsigned)((a.m + 16 * t.mb - 1) / (16 * t.mb)));
+    auto run = [&](auto fit, auto nt) {
+      qtts::launch(&w8a16_wide_kernel<XT, t.mb, t.nb, t.waves, t.cpw, t.cl, EPI, NORM, F8W, decltype(nt)::value, decltype(fit)::value>,
+                   grid, dim3(t.waves * 64), 0, a.st, a.qs, (const XT*)a.x, a.scale, (const XT*)a.bias, (const XT*)a.aux,
+                   (int)a.ldx, (int)a.m, (int)a.n, (int)(a.k / 64) << 8 | a.sdt, a.eps, (XT*)a.y, a.ldy,
+                   (const XT*)a.res, a.ldr);
+    };
     qtts::launch_by_policy<std::is_same<XT, bf16_t>::value>([&](auto nt) {
-      qtts::launch(&w8a16_wide_kernel<XT, t.mb, t.nb, t.waves, t.cpw, t.cl, EPI, NORM, F8W, decltype(nt)::value>, grid,
-                   dim3(t.waves * 64), 0, a.st, a.qs, (const XT*)a.x, a.scale, (const XT*)a.bias, (const XT*)a.aux,
-                   (int)a.ldx, (int)a.m, (int)a.n, a.sdt, a.eps, (XT*)a.y, a.ldy, (const XT*)a.res, a.ldr);
+      if (a.k == 64 * t.waves * t.cpw) run(std::true_type{}, nt);
+      else run(std::false_type{}, nt);
     });
   }
 }
@@ -368,10 +399,14 @@ template <typename XT, int EPI, bool F8W> inline bool launch_half(const HalfCfg&
   const dim3 grid((unsigned)((a.n + 15) / 16 * 2), 1, (unsigned)((a.m + 7) / 8));
 #define QTTS_HALF(W, UPW)                                                                                       \
   if (c.waves == W && c.upw == UPW) {                                                                           \
+    auto run = [&](auto fit, auto nt) {                                                                         \
+      qtts::launch(&w8a16_wide_half_kernel<XT, W, UPW, EPI, F8W, decltype(nt)::value, decltype(fit)::value>, grid, \
+                   dim3(W * 64), 0, a.st, a.qs, (const XT*)a.x, a.scale, (const XT*)a.bias, (int)a.ldx, (int)a.m, \
+                   (int)a.n, (int)(a.k / 128) << 8 | a.sdt, (XT*)a.y, a.ldy, (const XT*)a.res, a.ldr);          \
+    };                                                                                                          \
     qtts::launch_by_policy<std::is_same<XT, bf16_t>::value>([&](auto nt) {                                      \
-      qtts::launch(&w8a16_wide_half_kernel<XT, W, UPW, EPI, F8W, decltype(nt)::value>, grid, dim3(W * 64), 0, a.st, \
-                   a.qs, (const XT*)a.x, a.scale, (const XT*)a.bias, (int)a.ldx, (int)a.m, (int)a.n, a.sdt,     \
-                   (XT*)a.y, a.ldy, (const XT*)a.res, a.ldr);                                                   \
+      if (a.k == 128 * W * UPW) run(std::true_type{}, nt);                                                      \
+      else run(std::false_type{}, nt);                                                                          \
     });                                                                                                         \
     return true;                                                                                                \
   }

@@ -11,7 +11,7 @@ int qtts_launch_w8a16_wide(const void* x, int x_dtype, int64_t m, int64_t k, int
   const HalfCfg h = half_cfg(m, n, k);
   const int tile = wide_cfg(m, n, k, kWidePlain);
   if ((h.waves == 0 && tile < 0) || ldx > INT32_MAX) return 1;
-  const WideArgs a{x, m, ldx, qs, n, scale, sdt, bias, nullptr, 0.0f, res, ldr, y, ldy, st};
+  const WideArgs a{x, m, k, ldx, qs, n, scale, sdt, bias, nullptr, 0.0f, res, ldr, y, ldy, st};
   if (h.waves > 0) {
     bool ok;
     if (x_dtype == QTTS_BF16) ok = res ? launch_half<bf16_t, kEpiRes, false>(h, a) : launch_half<bf16_t, kEpiNone, false>(h, a);

@@ -9,7 +9,7 @@ int qtts_launch_fp8w_wide(const void* x, int x_dtype, int64_t m, int64_t k, int6
   const HalfCfg h = half_cfg(m, n, k);
   const int tile = wide_cfg(m, n, k, kWideFp8);
   if ((h.waves == 0 && tile < 0) || ldx > INT32_MAX) return 1;
-  const WideArgs a{x, m, ldx, (const int8_t*)qs, n, scale, QTTS_F32, bias, nullptr, 0.0f, nullptr, 0, y, ldy, st};
+  const WideArgs a{x, m, k, ldx, (const int8_t*)qs, n, scale, QTTS_F32, bias, nullptr, 0.0f, nullptr, 0, y, ldy, st};
   if (h.waves > 0) {
     const bool done = x_dtype == QTTS_BF16 ? launch_half<bf16_t, kEpiNone, true>(h, a) : launch_half<f16_t, kEpiNone, true>(h, a);
     return done ? qtts_check_launch("fp8w_wide_half") : 1;

@@ -10,7 +10,7 @@ int qtts_launch_w8a16_wide_fused(const void* x, int x_dtype, int64_t m, int64_t 
                                  void* y, int64_t ldy, hipStream_t st) {
   const int tile = wide_cfg(m, n, k, pair ? (nw ? kWideNormPair : kWidePair) : kWideNorm);
   if (tile < 0 || ldx > INT32_MAX) return 1;
-  const WideArgs a{x, m, ldx, qs, n, scale, sdt, bias, nw, eps, nullptr, 0, y, ldy, st};
+  const WideArgs a{x, m, k, ldx, qs, n, scale, sdt, bias, nw, eps, nullptr, 0, y, ldy, st};
   if (x_dtype == QTTS_BF16) {
     if (!pair) launch_wide<bf16_t, kEpiNone, true, false>(tile, a);
     else if (nw) launch_wide<bf16_t, kEpiPair, true, false>(tile, a);

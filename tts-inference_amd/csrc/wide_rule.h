@@ -1,4 +1,4 @@
-// Which calls the wide kernel (wide.h) takes, and in which tile.
+// Which calls the wide kernels (wide.h) take, and in which tile.
 #pragma once
 
 #include <stdint.h>
@@ -24,43 +24,45 @@ constexpr int kWideTileCount = (int)(sizeof(kWideTiles) / sizeof(kWideTiles[0]))
 
 // Whether the decode kernel's row parts (skinny.h) keep a call of 9 to 16 rows: on 65 to 128 strips their two parts make 256
 // workgroups of 8 staged rows, against this kernel's 128 at most.  Measured at N = 1040 .. 2048, us a call, decode kernel -> wide:
-// K = 6144 plain at 12 / 16 rows 5.64 / 5.60 -> 6.08 / 6.40, residual 6.17 / 6.19 -> 6.67 / 7.06; K = 2048 with the norm 4.81 -> 5.38,
-// with the activation 3.56 -> 3.86, residual 3.63 -> 3.88, plain the same; K = 1024 and 3072 0.2 to 0.6 faster, and
-// the norm with the activation 0.6 to 1.6 everywhere.  (The activation alone at K = 6144 has no decode form: 0.9 to 1.4 faster.)
+// K = 6144 plain at 12 / 16 rows 5.64 / 5.60 -> 6.08 / 6.40, residual 6.17 / 6.19 -> 6.67 / 7.06 (K = 4096 and 5120 alike: 0.3 to 2.1
+// slower); K = 2048 with the norm 4.81 -> 5.38, with the activation 3.56 -> 3.86, residual 3.63 -> 3.88, plain the same (K = 1536: norm 0.2
+// slower, the rest within 0.2); K <= 1024 and 2560 .. 3072 0.2 to 0.6 faster, and the norm with the activation 0.6 to 1.7 everywhere.
+// The activation alone at 3072 < K <= 4096: 1.1 to 1.9 slower on up to 64 strips too (longer K has no decode form: 0.8 to 1.4 faster).
 inline bool row_parts_keep(int64_t m, int64_t strips, int64_t k, int form) {
-  if (m > 16 || strips <= 64 || strips > 128 || form == kWideNormPair || (form == kWidePair && k > 4096)) return false;
-  return k > 3072 || (k > 1024 && k <= 2048);
+  if (m > 16 || strips > 128 || form == kWideNormPair) return false;
+  if (form == kWidePair && k > 3072) return k <= 4096;
+  return strips > 64 && (k > 3072 || (k > 1024 && k <= 2048));
 }
 
-// The tile of kWideTiles for the automatic choice of an [m, k] x [n, k] call on strip weights, or -1: 9 to 128 rows (8 and fewer stay with the
-// decode kernel, whose half strips and row staging are faster there; with the norm inside and K <= 1024 from 5
-// rows: 8 rows of the predictor's qkv 5.50 -> 5.00 us, of its gate_up with the activation 6.59 -> 5.65) where K is a built
-// product of waves and chunks and one of the built tiles covers the call in a single round of
-// workgroups on the 256 compute units.  Of those tiles the one that reads the fewest bytes a workgroup:
+// The tile of kWideTiles for the automatic choice of an [m, k] x [n, k] call on strip weights, or -1: 9 to 128 rows (8 and
+// fewer stay with the decode kernel, whose half strips and row staging are faster there; with the norm inside and K <= 1024 from 5
+// rows: 8 rows of the predictor's qkv 5.50 -> 5.00 us, of its gate_up with the activation 6.59 -> 5.65) and 512 < K <= 6144
+// (shorter K within 0.2 us of the kernels that have it, either way, on wide weights; longer K would not fit the built runs),
+// where one of the built tiles covers the call in a single round of workgroups on the 256 compute units.
+// The waves share the K / 64 chunks, so that every K takes the group of tiles with the shortest runs that hold it: 2 chunks a
+// wave up to K = 1024, up to K = 2048 16 waves of 2 on more than 128 strips and 8 of 4 on fewer (32 rows: talker qkv 4.49 against
+// 4.84 us, o_proj + residual 4.43 against 4.19), 8 waves of 6 up to 3072, 16 of 6 beyond.  Measured off the tiles' full runs,
+// former automatic choice -> this, plain, N = 2048, 27 / 48 / 100 rows: K = 1088 5.80 / 6.14 / 6.30 -> 3.16 / 3.61 / 4.47, 1984 6.07 /
+// 7.57 / 7.76 -> 3.63 / 4.18 / 5.08, 2560 7.80 / 7.57 -> 4.09 / 4.89, 5120 9.03 / 8.85 -> 6.12 / 7.16.
+// Of the group's tiles the one that reads the fewest bytes a workgroup:
 // a second round costs more than any tile's extra bytes (the talker's gate_up past 32 rows, 512 workgroups,
-// 12.9 us at 48 rows against the tile kernel's 11.7).  K = 2048 runs 16 waves of 2 chunks on more than 128
-// strips and 8 of 4 on fewer (32 rows: talker qkv 4.49 against 4.84 us, o_proj + residual 4.43 against 4.19).
-// norm: with the RMSNorm inside, every workgroup repeats its rows' normalization, so the tile of the
+// 12.9 us at 48 rows against the tile kernel's 11.7).
+// With the norm inside every workgroup repeats its rows' normalization, so the tile of the
 // fewest rows is taken and at most 32768 elements (16 rows of 2048): past them the norm's own launch
 // (about 2.7 us) is cheaper (talker gate_up at 32 rows 12.0 inside against 8.3 + 2.7; predictor gate_up
 // at 128 10.7 against 7.5 + 2.9, and inside up to 64 rows, 7.48 against 8.6).
-// pair: a gate_up weight with its activation.  K = 1024 past 48 rows: plain and residual calls stay with the
-// tile kernel, whose result the automatic choice is held to bit for bit there (they would
-// gain 0.1-0.9 us a call).
+// K <= 1024 past 48 rows: plain and residual calls stay with the kernels that had them before this one, because the
+// automatic choice is held to the tile kernel's bits there (they would gain 0.1-3.8 us a call).
 inline int wide_cfg(int64_t m, int64_t n, int64_t k, int form) {
-  const bool norm = (form & (kWideNorm | kWideNormPair)) != 0, pair = (form & (kWidePair | kWideNormPair)) != 0;
-  if (k == 1024 && m > 48 && !norm && !pair) return -1;
-  if (m < (norm && k <= 1024 ? 5 : 9) || m > 128 || n <= 0 || n > (1 << 30)) return -1;
-  const int64_t strips = (n + 15) / 16;
+  const bool norm = (form & (kWideNorm | kWideNormPair)) != 0;
+  if ((form == kWidePlain || form == kWideFp8) && k <= 1024 && m > 48) return -1;
+  if (m < (norm && k <= 1024 ? 5 : 9) || m > 128 || n <= 0 || n > (1 << 30) || k % 64 != 0 || k <= 512 || k > 6144) return -1;
+  const int64_t strips = (n + 15) / 16, chunks = k / 64;
   if (row_parts_keep(m, strips, k, form)) return -1;
   int waves, cpw;
-  switch (k) {
-    case 1024: waves = 8, cpw = 2; break;
-    case 2048: waves = strips > 128 ? 16 : 8, cpw = strips > 128 ? 2 : 4; break;
-    case 3072: waves = 8, cpw = 6; break;
-    case 6144: waves = 16, cpw = 6; break;
-    default: return -1;
-  }
+  if (chunks <= 16) waves = 8, cpw = 2;
+  else if (chunks <= 32) waves = strips > 128 ? 16 : 8, cpw = strips > 128 ? 2 : 4;
+  else waves = chunks <= 48 ? 8 : 16, cpw = 6;
   int best = -1;
   int64_t best_cost = 0;
   for (int i = 0; i < kWideTileCount; ++i) {
@@ -80,17 +82,15 @@ inline int wide_cfg(int64_t m, int64_t n, int64_t k, int form) {
 
 struct HalfCfg { int waves, upw; };  // waves == 0: not this kernel
 
-// Half strips in 8-row parts (wide.h): where the strips times two times the parts make one round of at most 256
-// workgroups (up to 16 rows on 64 strips, 8 on 128) and K is a built product.  From 5 rows: below,
+// Half strips in 8-row parts (wide.h): from 5 rows, 512 < K <= 6144 and K % 128 == 0, where the strips times two times the parts make one
+// round of at most 256 workgroups: 16 rows on 64 strips, 8 on 128.  The waves share the K / 128 units as the chunks above.  Below 5 rows
 // skinny.h stages fewer rows, and whole steps run faster on it: 10 predictor layers at 2 / 4 rows 155.1 / 165.3 us
 // against 160.7 / 167.9 with these (8 rows: 187.1 against 177.9), 4 talker layers 85.9 / 91.6 against 87.6 / 92.0
 // (8 rows: 107.0 against 103.0).
 inline HalfCfg half_cfg(int64_t m, int64_t n, int64_t k) {
-  if (m < 5 || n < 1 || (n + 15) / 16 * 2 * ((m + 7) / 8) > 256) return HalfCfg{0, 0};
-  if (k == 2048) return HalfCfg{8, 2};
-  if (k == 3072) return HalfCfg{8, 3};
-  if (k == 6144) return HalfCfg{12, 4};
-  return HalfCfg{0, 0};
+  if (m < 5 || n < 1 || (n + 15) / 16 * 2 * ((m + 7) / 8) > 256 || k % 128 != 0 || k <= 512 || k > 6144) return HalfCfg{0, 0};
+  if (k <= 2048) return HalfCfg{8, 2};
+  return k <= 3072 ? HalfCfg{8, 3} : HalfCfg{12, 4};
 }
 
 // Whether the automatic choice runs a plain (or residual) call on the wide kernels.
