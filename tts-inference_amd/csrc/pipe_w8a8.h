@@ -114,10 +114,21 @@ __global__ __launch_bounds__(NW * 64) void w8a8_pipe_kernel(
   const int kc0 = split * cps;
   const int nk = min(cps, nchunks - kc0);
 
-  // Epilogue operands first, as raw bits (loads the compiler will not sink).
+  // Epilogue operands first, as raw bits (loads the compiler will not sink).  With read-ahead on the largest tiles
+  // (kPark) they meet two operand sets in the registers: one row and one column a thread, parked in LDS until the end.
+  // Held in registers they spilled 36-49 a lane into the K loop (now 0, fp8 3); gate_up at 2048 rows, us: fp8 111.0 -> 74.3,
+  // int8 83.6 -> 69.4, int8 row-major 95.6 -> 88.9; at 1024 72.7 -> 47.0, 53.2 -> 44.9, 64.3 -> 59.9.
+  constexpr bool kPark = PF && NW == 8 && BM * BN >= 128 * 256;
+  static_assert(!kPark || (BM <= NW * 64 && BN <= NW * 64 && P * SB + 64 + 4 * (BM + 2 * BN) <= kLdsBytes), "a thread each");
+  __shared__ uint32_t epi_sx[kPark ? BM : 1], epi_sw[kPark ? BN : 1], epi_bi[kPark ? BN : 1];
   uint32_t sxb[MB], swb[NB][4], bib[NB][4];
-  {
-    const OT* bsrc = bias ? bias : y;
+  const OT* bsrc = bias ? bias : y;
+  if constexpr (kPark) {
+    const int n = min(n0 + tid, N - 1);
+    sxb[0] = load_out_bits((const float*)sx + min(m0 + tid, M - 1));
+    swb[0][0] = load_out_bits((const float*)sw + n);
+    bib[0][0] = load_out_bits(bsrc + n);
+  } else {
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb)
       sxb[mb] = __hip_atomic_load((uint32_t*)sx + min(m0 + mb * 16 + c16, M - 1), __ATOMIC_RELAXED,
@@ -170,7 +181,7 @@ __global__ __launch_bounds__(NW * 64) void w8a8_pipe_kernel(
   // A stage's operands: every activation half of the tile, and this wave's weight halves.
   struct Ops { i32x4_t x0[MB], x1[MB], w0[NB], w1[NB]; };
   const int xoff0 = c16 * 128 + 16 * swizzle8(c16, Kind::col(g, 0) >> 4);
-  const int xoff1 = c16 * 128 + 16 * swizzle8(c16, Kind::col(g, 1) >> 4);
+  const int xoff1 = xoff0 ^ Kind::col(0, 1);  // (the halves' pieces differ in one bit, and so do their positions)
   auto read = [&](Ops& o, const uint8_t* stage) __attribute__((always_inline)) {
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb) {
@@ -193,6 +204,15 @@ __global__ __launch_bounds__(NW * 64) void w8a8_pipe_kernel(
 
   for (int p = 0; p < P - 1; ++p)
     if (p < nk) issue(ring + p * SB, p);
+  if constexpr (kPark) {
+    if (tid < BM) epi_sx[tid] = sxb[0];
+    if (tid < BN) {
+      epi_sw[tid] = swb[0][0];
+      epi_bi[tid] = bib[0][0];
+    }
+    wait_lgkmcnt0();
+    barrier_only();
+  }
   if constexpr (!PF) {
     // Stage i: wait for this wave's loads of stage i (up to P-2 later stages may stay in
     // flight), barrier, issue stage i+P-1, read and consume stage i.
@@ -268,14 +288,15 @@ __global__ __launch_bounds__(NW * 64) void w8a8_pipe_kernel(
     float swv[4], biv[4];
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
-      swv[t] = __uint_as_float(swb[nb][t]);
-      biv[t] = out_bits_to_f32<OT>(bib[nb][t]);
+      const int col = (wave * NB + nb) * 16 + 4 * g + t;
+      swv[t] = __uint_as_float(kPark ? epi_sw[kPark ? col : 0] : swb[nb][t]);
+      biv[t] = out_bits_to_f32<OT>(kPark ? epi_bi[kPark ? col : 0] : bib[nb][t]);
     }
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb) {
       const int m = m0 + mb * 16 + c16;
       if (m >= M) continue;
-      const float sxv = __uint_as_float(sxb[mb]);
+      const float sxv = __uint_as_float(kPark ? epi_sx[kPark ? mb * 16 + c16 : 0] : sxb[mb]);
       OT* yr = y + (int64_t)m * ldy;
       float v[4];
 #pragma unroll
