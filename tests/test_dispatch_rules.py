@@ -124,3 +124,23 @@ int main() {
             assert waves <= k // 64 <= waves * cpw and (k // 64 > 3 * 16 or waves * cpw <= 48), k
         assert (units > 0) == (k % 128 == 0 and 512 < k <= 6144), k
         assert not units or k // 128 <= units, k
+
+
+def test_half_strips_take_one_round_of_workgroups(tmp_path):
+    """Two half strips times the 8-row parts, at most 256: the last row of each line of strips, and the first past it."""
+    rows = _run(tmp_path, """
+#include <stdio.h>
+#include "wide_rule.h"
+using namespace qtts;
+int main() {
+  const int ns[] = {1, 16, 17, 64, 200, 512, 1000, 1024, 2048, 2049};
+  for (int n : ns)
+    for (int m = 1; m <= 1100; ++m) printf("%d %d %d\\n", n, m, half_cfg(m, n, 2048).waves);
+}
+""")
+    last = {}
+    for n, m, waves in rows:
+        if waves:
+            assert m >= 5, (n, m)
+            last[n] = m
+    assert last == {1: 1024, 16: 1024, 17: 512, 64: 256, 200: 72, 512: 32, 1000: 16, 1024: 16, 2048: 8}

@@ -405,9 +405,11 @@ def test_wide_fp8_codes(ops, m, n, k):
     assert_close(ops.fp8w_gemm_strips(x, ops.fp8w_strips(q), n, s), _ref64(x, q.float(), s, None), f"wide fp8 {m} {n} {k}")
 
 
-# (m, n, k) of the half strips: idle waves (K / 128 below the waves), runs that differ by one, whole ones; ragged rows and columns
+# (m, n, k) of the half strips: idle waves (K / 128 below the waves), runs that differ by one, whole ones; ragged rows and columns;
+# more rows of fewer strips, to the last row part that one round holds
 HALF = [(5, 200, 640), (8, 2048, 768), (7, 1000, 1152), (16, 1024, 1920), (8, 2040, 2048), (12, 1000, 2176), (16, 1024, 3072),
-        (13, 1000, 5120), (8, 2048, 6016), (5, 2048, 6144)]
+        (13, 1000, 5120), (8, 2048, 6016), (5, 2048, 6144), (17, 512, 640), (31, 500, 2048), (72, 200, 1024), (65, 195, 3072),
+        (256, 64, 1920), (1024, 16, 2048), (1001, 9, 6144)]
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])

@@ -14,7 +14,7 @@
 //    epilogue's scale and bias are fetched first, so a call costs one memory round
 //    trip.  Waves meet in LDS; workgroups that split K further meet through the
 //    workspace (splitk.h) with no second launch.
-//  * wide (9-128 rows where one round of workgroups covers the call): wide.h.
+//  * wide (5-128 rows, more on very few strips, where one round of workgroups covers the call): wide.h, wide_rule.h.
 //  * tile (M > 16, prefill rows): LDS-tiled bf16 MFMA GEMM, BM x 128 x 64 tiles,
 //    4 waves in 2x2, double-buffered LDS; the weight tile is dequantized to bf16 on
 //    its way into LDS.

@@ -1,4 +1,4 @@
-// The wide kernel (wide.h) on e4m3 codes: fp8 weight-only calls of 9 to 128 rows.
+// The wide kernels (wide.h) on e4m3 codes: the fp8 weight-only calls that wide_rule.h names.
 #include "wide.h"
 
 using namespace qtts;

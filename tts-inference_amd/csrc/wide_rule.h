@@ -83,7 +83,11 @@ inline int wide_cfg(int64_t m, int64_t n, int64_t k, int form) {
 struct HalfCfg { int waves, upw; };  // waves == 0: not this kernel
 
 // Half strips in 8-row parts (wide.h): from 5 rows, 512 < K <= 6144 and K % 128 == 0, where the strips times two times the parts make one
-// round of at most 256 workgroups: 16 rows on 64 strips, 8 on 128.  The waves share the K / 128 units as the chunks above.  Below 5 rows
+// round of at most 256 workgroups: 8 rows on 128 strips, 16 on 64, 32 on 32, and so on to 1024 rows on one.  Measured over that
+// whole line, no call slower than with the former choice; us a call at K = 1024 / 2048 / 6144, plain: N = 2048, 8 rows 3.80 / 3.74 / 5.35 ->
+// 3.03 / 3.49 / 4.62; N = 1024, 16 rows 3.79 / 3.49 / 5.00 -> 3.05 / 3.15 / 4.26; N = 512, 32 rows 3.79 / 3.47 / 4.93 -> 3.04 / 3.15 / 4.11; N = 200,
+// 72 rows 5.94 / 6.53 / 8.68 -> 3.06 / 3.15 / 4.19; N = 64, 256 rows 5.84 / 6.41 / 12.10 -> 3.05 / 3.14 / 3.97; N = 16, 1024 rows 8.35 / 9.50 /
+// 13.03 -> 3.01 / 3.10 / 3.97 (e4m3 codes alike, the residual 0.1 to 2 more saved).  The waves share the K / 128 units as the chunks above.  Below 5 rows
 // skinny.h stages fewer rows, and whole steps run faster on it: 10 predictor layers at 2 / 4 rows 155.1 / 165.3 us
 // against 160.7 / 167.9 with these (8 rows: 187.1 against 177.9), 4 talker layers 85.9 / 91.6 against 87.6 / 92.0
 // (8 rows: 107.0 against 103.0).
