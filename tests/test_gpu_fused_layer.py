@@ -335,8 +335,8 @@ def test_tile_silu_pair_epilogue(ops, m, n, k, dtype):
             assert torch.equal(ops.w8a16_gate_up_silu_strips(x, qs, n, s, bias, **kw), want)
 
 
-# (m, n, k): row edges of the 16-row blocks (with 5 rows for the norm inside), ragged columns, each built K
-WIDE = [(5, 4096, 1024), (9, 4096, 1024), (16, 100, 1024), (17, 6144, 1024), (33, 4096, 1024), (48, 1040, 1024),
+# (m, n, k): row edges of the 16-row blocks (with 5 to 8 rows for the norm inside), ragged columns, each built K
+WIDE = [(5, 4096, 1024), (6, 4096, 1024), (7, 6144, 1024), (8, 1024, 1024), (9, 4096, 1024), (16, 100, 1024), (17, 6144, 1024), (33, 4096, 1024), (48, 1040, 1024),
         (65, 6144, 1024), (96, 6144, 1024), (128, 6144, 1024), (9, 12288, 2048), (31, 12288, 2048), (47, 4096, 2048),
         (128, 4096, 2048), (27, 2048, 2048), (127, 2048, 2048), (12, 1000, 3072), (97, 1024, 3072), (13, 2048, 6144),
         (32, 2048, 6144), (64, 2048, 6144)]
@@ -352,11 +352,12 @@ def _ref64(h, q, s, b):
     return (y if b is None else y + b.double()).cpu().numpy()
 
 
-def _bar_product(y, gate, up, what):
+def _bar_product(y, gate, up, what, dtype):
     """The GEMM bar carried through silu(g) * u to first order: |d silu| <= 1.1 |dg|, half an output ulp each for the
-    roundings of g, u and silu(g) in between."""
+    roundings of g, u and silu(g) in between (dtype's ulp: 7 fraction bits, or 10 down to 2^-24)."""
     def half(v):
-        return 2.0 ** (np.floor(np.log2(np.maximum(np.abs(v), 1e-30))) - 7) / 2
+        e = np.floor(np.log2(np.maximum(np.abs(v), 1e-30)))
+        return 2.0 ** (e - 7 if dtype == torch.bfloat16 else np.maximum(e, -14) - 10) / 2
     rms_g, rms_u = (np.sqrt(np.mean(v * v)) for v in (gate, up))
     silu = gate / (1 + np.exp(-gate))
     dg, du = 1e-2 * rms_g + half(gate), 1e-2 * rms_u + half(up)
@@ -392,7 +393,26 @@ def test_wide_calls(ops, m, n, k, dtype):
         for h, kw in ((x, {}), (hn, {"prologue": ops.PRO_RMS_NORM, "norm_weight": nw})):
             full = _ref64(h, q, s, b)
             act = ops.w8a16_gate_up_silu_strips(x, qs, n, s, b, **kw)
-            _bar_product(act.double().cpu().numpy(), full[:, : n // 2], full[:, n // 2:], what + str(list(kw)))
+            _bar_product(act.double().cpu().numpy(), full[:, : n // 2], full[:, n // 2:], what + str(list(kw)), dtype)
+
+
+# (m, n, k): the plain (or norm) call and the one with the activation take the same waves over the same K
+@pytest.mark.parametrize("norm,m,n,k", [(False, 33, 4096, 1024), (False, 48, 1024, 704), (False, 31, 12288, 2048), (False, 27, 12288, 1536),
+                                        (False, 17, 6144, 1088), (False, 33, 2048, 2048), (False, 17, 2048, 3072), (False, 32, 2048, 6144),
+                                        (True, 5, 4096, 1024), (True, 8, 4096, 960), (True, 33, 4096, 1024), (True, 64, 6144, 1024),
+                                        (True, 12, 4096, 2048), (True, 31, 4096, 1984)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("sdt", [None, torch.float32])
+def test_wide_silu_pair_bits(ops, norm, m, n, k, dtype, sdt):
+    """The wide kernel's activation: bit for bit silu_mul of its call without it (gate, up and silu(gate) each rounded once)."""
+    q, s, qs = _weights(ops, n, k, dtype, 7)
+    s = s if sdt is None else (s.float() * (1 + 2.0 ** -13)).to(sdt)
+    g = torch.Generator(device="cuda").manual_seed(m * 3 + k)
+    x = torch.randn(m, k, device="cuda", generator=g).to(dtype)
+    kw = {"prologue": ops.PRO_RMS_NORM, "norm_weight": (1 + 0.1 * torch.randn(k, device="cuda", generator=g)).to(dtype)} if norm else {}
+    for bias in (None, torch.randn(n, device="cuda", generator=g).to(dtype)):
+        full = ops.w8a16_fused_gemm_strips(x, qs, n, s, bias, **kw) if norm else ops.w8a16_gemm_strips(x, qs, n, s, bias)
+        assert torch.equal(ops.w8a16_gate_up_silu_strips(x, qs, n, s, bias, **kw), ops.silu_mul(full)), (m, n, k, dtype)
 
 
 @pytest.mark.parametrize("m,n,k", [(9, 4096, 1024), (33, 6144, 1024), (47, 4096, 2048), (97, 1024, 3072), (64, 2048, 6144)] + WIDE_K)

@@ -14,7 +14,7 @@ import torch
 
 pytestmark = pytest.mark.gpu
 
-SHAPES = [(2048, 2048), (2048, 6144), (12288, 2048), (1024, 3072), (96, 512)]
+SHAPES = [(2048, 2048), (2048, 6144), (12288, 2048), (1024, 3072), (4096, 1024), (96, 512)]
 ROWS = (1, 2, 3, 4, 5, 8, 12, 16, 40)
 
 
@@ -67,9 +67,9 @@ def test_w8a16_stream_flag_same_bits(ops, n, k):
             _same(lambda f: ops.w8a16_gemm(x, q, s, b, ops.ALGO_AUTO | f), f"{what} row-major")
 
 
-@pytest.mark.parametrize("n,k", [(4096, 2048), (12288, 2048), (2048, 6144), (96, 512)])
+@pytest.mark.parametrize("n,k", [(4096, 2048), (12288, 2048), (2048, 6144), (4096, 1024), (96, 512)])
 def test_fused_forms_stream_flag_same_bits(ops, n, k):
-    for m in (1, 2, 4, 8, 12):
+    for m in (1, 2, 4, 5, 8, 12, 40):
         w, b = _weights(ops, n, k, seed=3 * n + k)
         q, s = ops.pack_int8(w, torch.bfloat16)
         qs = ops.to_strips(q)
@@ -89,7 +89,7 @@ def test_fused_forms_stream_flag_same_bits(ops, n, k):
         _same(lambda f: ops.w8a16_silu_mul_gemm_strips(gu, qs, n, s, b, f), f"{what} silu_mul")
 
 
-@pytest.mark.parametrize("n,k", [(2048, 2048), (2048, 6144), (1024, 3072)])
+@pytest.mark.parametrize("n,k", [(2048, 2048), (2048, 6144), (1024, 3072), (4096, 1024)])
 def test_fp8_and_int8_stream_flag_same_bits(ops, n, k):
     w, b = _weights(ops, n, k, seed=7 * n + k)
     qf, sf = ops.pack_fp8(w)
