@@ -762,7 +762,7 @@ def run_traffic_probe(args, torch, ops):
 def run_prefill_probe(args, torch, ops):
     """Kernels for a rocprofv3 --pmc pass over the prefill tile kernel: configs[3]'s gate_up
     (12288 x 2048) at M = 1024, launched eagerly 8 times each (after 3 warm-up launches) as the automatic tile
-    (8 waves, 128 x 256), as the 4-wave 128 x 128 tile (3 stages, no read-ahead, no split), and as F.linear on the
+    (8 waves, 128 x 384), as the 4-wave 128 x 128 tile (3 stages, no read-ahead, no split), and as F.linear on the
     bf16 weight (hipBLASLt)."""
     from qtts_amd import _lib
     ops.reserve_workspace(torch.device("cuda"), 64 << 20)

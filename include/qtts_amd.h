@@ -246,10 +246,13 @@ int qtts_rms_norm(const void* x, int x_dtype, int64_t m, int64_t k, int64_t ldx,
  *   residual: [m, n] of x_dtype, row stride ldr, or NULL; y = dtype(f32(residual) +
  *   f32(linear)), the linear rounded to x_dtype first, as `residual + o_proj(...)`
  *   (talker.py:270-271).  residual may be y itself (an in-place hidden-state update).
- * Fused into the GEMM launch (prologue computed while the activation rows are staged,
- * residual added in the epilogue): SiLU for m == 1, RMSNorm for m <= 16 (without a
- * residual and without split-K), the residual for m <= 16 (9-16 rows in two row parts of
- * 8 with one split) and up to 64 on half strips (row parts of 8).  Otherwise the separate kernels run around qtts_w8a16_gemm_strips,
+ * Fused into the GEMM launch by the automatic choice (prologue computed while the activation
+ * rows are staged, residual added in the epilogue): SiLU for m == 1; RMSNorm without a residual
+ * for m <= 16 (without split-K) and for up to 128 rows where one round of workgroups covers the
+ * call and normalizes at most 32768 elements each (512 < k <= 2048); the residual at every m on
+ * the decode, wide and tile kernels (9-16 rows in two row parts of 8 with one split; not on the
+ * decode kernel's 17-32 rows of small weights).  Otherwise, and for requested algorithms past
+ * the decode rows, the separate kernels run around qtts_w8a16_gemm_strips,
  * through the workspace.  SiLU and the residual give the same bits either way; a fused
  * RMSNorm stages dtype((x * inv) * w) as qtts_rms_norm does, with its sum of squares in
  * another order.  scale_dtype: x_dtype or fp32 for the fused launches (any
@@ -265,11 +268,13 @@ int qtts_w8a16_fused_gemm_strips(const void* x, int x_dtype, int64_t m, int64_t 
  *   h = x (QTTS_PRO_NONE) or qtts_rms_norm(x, norm_weight, eps) (QTTS_PRO_RMS_NORM),
  *   g | u = w8a16_linear(h) (qs: the fused [n, k] gate_up weight, gate rows first),
  *   act[r, c] = dtype(dtype(silu(g[r, c])) * u[r, c])   for c < n / 2
- * with the rounding of qtts_w8a16_fused_gemm_strips followed by qtts_silu_mul.  Up to 16
- * decode rows with n % 32 == 0 run as ONE launch (a workgroup holds gate strip s and up
- * strip s + n/32 and writes the activation from its epilogue; the gate_up output is
- * never stored); otherwise the prologue, the GEMM and qtts_silu_mul run in turn through
- * the workspace.  No counterpart in the reference, which stores gate_up and runs the
+ * with the rounding of qtts_w8a16_fused_gemm_strips followed by qtts_silu_mul.  With
+ * n % 32 == 0 the activation is in the epilogue of ONE launch (a workgroup holds gate rows and
+ * the matching up rows; the gate_up output is never stored): up to 16 decode rows with the
+ * RMSNorm inside, past them by the automatic choice on the wide kernel (RMSNorm inside as
+ * above) or the tile kernel (RMSNorm first, a launch of its own).  Otherwise the prologue,
+ * the GEMM and qtts_silu_mul run in turn through the workspace, which every call past the
+ * decode kernel's (16 rows, k <= 4096) must bring.  No counterpart in the reference, which stores gate_up and runs the
  * activation as two more kernels.  x: [m, k] bf16 / fp16, 16-byte aligned rows, k % 64 == 0.
  * act: [m, n / 2], row stride ldact.  Workspace: qtts_workspace_bytes(QTTS_OP_W8A16_FUSED). */
 int qtts_w8a16_gate_up_silu_strips(const void* x, int x_dtype, int64_t m, int64_t k, int64_t ldx,

@@ -15,7 +15,8 @@
 // Measured on the talker's linears (three weights in turn, us, pipe_w8a8.h's choice -> this one): int8
 // gate_up at 512 / 1024 / 1500 / 2048 rows 22.9 / 41.3 / 58.2 / 61.0 -> 19.0 / 29.5 / 48.8 / 54.5, qkv at 1024 /
 // 1500 15.1 / 22.4 -> 14.0 / 18.4, o_proj at 1500 / 2048 14.4 / 15.5 -> 13.5 / 14.4, down_proj 32.0 / 33.8 -> 28.0 /
-// 29.4; fp8 gate_up at 1024 / 1500 42.0 / 59.6 -> 36.6 / 57.3, qkv at 1500 22.9 -> 21.3.  An ablation of
+// 29.4; fp8 gate_up at 1024 / 1500 42.0 / 59.6 -> 36.6 / 57.3, qkv at 1500 22.9 -> 21.3 (at 2048 rows all four fp8
+// linears fill whole rounds of pipe_w8a8.h's tiles and stay there).  An ablation of
 // gate_up at 1024 rows (int8, 31.3 us under it): 26.5 without the global loads, 29.9 without the LDS reads, 23.6
 // without the MFMAs: no single one bounds it; about 10 us are the launch, the first stages and the
 // 25 MB of output that a single round writes at its end.

@@ -16,9 +16,11 @@
 //    GEMM writes t into the workspace: y may be the residual itself).
 //  * qtts_launch_w8a16_fused: one skinny launch with the prologue computed while the
 //    activation row is staged in LDS and the residual added in the epilogue
-//    (skinny.h: PRO, RES) when the call allows it; past the decode rows the separate
-//    prologue and one tile launch with the residual in its epilogue (tile_fused.hip);
-//    otherwise the separate kernels around the plain W8A16 GEMM.  Fused: SiLU for one row (for two rows it no longer
+//    (skinny.h: PRO, RES) when the call allows it; one wide launch with the RMSNorm or
+//    the residual (wide.h) where its rule takes the call (wide_rule.h: 5-128 rows that one round of
+//    workgroups covers); past both the separate prologue and one tile launch with the residual in
+//    its epilogue (tile_fused.hip); otherwise the separate kernels around the plain W8A16
+//    GEMM.  Fused on the decode kernel: SiLU for one row (for two rows it no longer
 //    hides under the weight stream: talker down 9.4 us fused against 9.0 us for the
 //    two passes at M = 2; 7.0 against 9.1 us at M = 1); RMSNorm for up to 16 rows without
 //    a split-K (every workgroup needs the whole row's sum); the residual for up to 16
@@ -549,10 +551,10 @@ int64_t qtts_w8a16_silu_ws_bytes(int64_t m, int64_t n, int64_t k, int algo, int 
 // act = silu(gate) * up of GatedMLP's gate_up_proj(prologue(x)) on strip weights
 // (qtts/layers/activation.py:142-147): x [m, k]; prologue none or RMSNorm (nw, eps);
 // qs the fused [n, k] gate_up weight (gate rows then up rows, n % 2 == 0); act [m, n/2]
-// with row stride ldact.  Up to 16 decode rows (n % 32 == 0): one launch, the activation
-// in the GEMM's epilogue.  Past them (automatic choice, n % 32 == 0) the norm, then one tile
-// launch with the activation in its epilogue (tile_fused.hip).  Otherwise the norm, the GEMM
-// into the workspace and silu_mul run one after another.
+// with row stride ldact.  n % 32 == 0: up to 16 decode rows one launch with the norm and the
+// activation, the wide kernel's (wide_rule.h) or the decode kernel's; past them (automatic choice) one wide
+// launch with both, else the norm, then one wide or tile launch (tile_fused.hip) with the activation
+// in its epilogue.  Otherwise the norm, the GEMM into the workspace and silu_mul run one after another.
 int qtts_launch_w8a16_gate_up_silu(const void* x, int x_dtype, int64_t m, int64_t k, int64_t ldx, int pro,
                                    const void* nw, float eps, const int8_t* qs, int64_t n, const void* scale, int sdt,
                                    const void* bias, void* act, int64_t ldact, int algo, void* ws, int64_t ws_bytes,

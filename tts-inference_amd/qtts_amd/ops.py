@@ -786,9 +786,10 @@ def w8a16_gate_up_silu_strips(x: torch.Tensor, qs: torch.Tensor, n: int, scale: 
                               norm_weight: torch.Tensor | None = None, eps: float = 1e-6,
                               algo: int = ALGO_AUTO) -> torch.Tensor:
     """``F.silu(gate) * up`` of GatedMLP's fused ``gate_up_proj(prologue(x))`` (qtts/layers/activation.py:
-    142-147) on an int8 strip-layout ``[n, K]`` gate_up weight; returns ``[..., n // 2]``.  Up to 8
-    rows run as one kernel with the activation in the GEMM's epilogue (the gate_up output is never
-    stored).  ``prologue``: PRO_NONE or PRO_RMS_NORM (with ``norm_weight`` and ``eps``)."""
+    142-147) on an int8 strip-layout ``[n, K]`` gate_up weight; returns ``[..., n // 2]``.  With
+    ``n % 32 == 0`` the automatic choice applies the activation in the GEMM's epilogue at every row count
+    (the gate_up output is never stored), up to 16 rows and where one round of workgroups covers the call
+    with the norm inside too.  ``prologue``: PRO_NONE or PRO_RMS_NORM (with ``norm_weight`` and ``eps``)."""
     shape = x.shape
     a = _flatten(x)
     rows, k = a.shape
