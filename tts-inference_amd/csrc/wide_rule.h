@@ -51,8 +51,9 @@ inline bool row_parts_keep(int64_t m, int64_t strips, int64_t k, int form) {
 // fewest rows is taken and at most 32768 elements (16 rows of 2048): past them the norm's own launch
 // (about 2.7 us) is cheaper (talker gate_up at 32 rows 12.0 inside against 8.3 + 2.7; predictor gate_up
 // at 128 10.7 against 7.5 + 2.9, and inside up to 64 rows, 7.48 against 8.6).
-// K <= 1024 past 48 rows: plain and residual calls stay with the kernels that had them before this one, because the
-// automatic choice is held to the tile kernel's bits there (they would gain 0.1-3.8 us a call).
+// K <= 1024 past 48 rows: plain and residual calls stay with the tile kernel and the decode kernel's half strips, because the
+// automatic choice is held to the tile kernel's bits there (64 rows of 4096 x 1024; they would gain 0.1-3.8 us a call), and
+// e4m3 codes with them, one line for both.
 inline int wide_cfg(int64_t m, int64_t n, int64_t k, int form) {
   const bool norm = (form & (kWideNorm | kWideNormPair)) != 0;
   if ((form == kWidePlain || form == kWideFp8) && k <= 1024 && m > 48) return -1;
