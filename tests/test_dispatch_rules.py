@@ -144,3 +144,33 @@ int main() {
             assert m >= 5, (n, m)
             last[n] = m
     assert last == {1: 1024, 16: 1024, 17: 512, 64: 256, 200: 72, 512: 32, 1000: 16, 1024: 16, 2048: 8}
+
+
+def test_decode_kernel_keeps_few_strips_that_half_strips_cannot_split(tmp_path):
+    """9-16 rows on up to 64 strips with K an odd multiple of 64 (no half strips): the decode kernel from where it measured faster,
+    K > 3072, or K > 1280 with the norm inside; whole units of 128 and 17 rows go on as before."""
+    rows = _run(tmp_path, """
+#include <stdio.h>
+#include <initializer_list>
+#include "wide_rule.h"
+using namespace qtts;
+int main() {
+  const int ks[] = {1088, 1344, 1984, 2048, 3008, 3136, 3200, 4032, 6080}, ns[] = {224, 1024}, ms[] = {9, 16, 17};
+  for (int k : ks)
+    for (int n : ns)
+      for (int m : ms)
+        for (int form : {kWidePlain, kWideFp8, kWideNorm, kWidePair})
+          printf("%d %d %d %d %d\\n", k, n, m, form, wide_cfg(m, n, k, form) >= 0 || (form != kWideNorm && form != kWidePair && half_cfg(m, n, k).waves));
+}
+""")
+    plain, norm, pair, fp8 = 1, 2, 4, 16
+    assert len(rows) == 9 * 2 * 3 * 4
+    for k, n, m, form, taken in rows:
+        odd = k % 128 != 0 and m <= 16
+        if form in (plain, fp8):
+            want = not (odd and k > 3072)
+        elif form == norm:
+            want = k <= 2048 and not (odd and k > 1280)
+        else:
+            want = not (3072 < k <= 4096 and m <= 16)
+        assert taken == want, (k, n, m, form)

@@ -22,16 +22,20 @@ constexpr WideTile kWideTiles[] = {
     {1, 1, 16, 6, 4, 21}, {1, 2, 16, 6, 4, 21}};
 constexpr int kWideTileCount = (int)(sizeof(kWideTiles) / sizeof(kWideTiles[0]));
 
-// Whether the decode kernel's row parts (skinny.h) keep a call of 9 to 16 rows: on 65 to 128 strips their two parts make 256
-// workgroups of 8 staged rows, against this kernel's 128 at most.  Measured at N = 1040 .. 2048, us a call, decode kernel -> wide:
+// Whether the decode kernel keeps a call of 9 to 16 rows on up to 128 strips, where this kernel has at most 128 workgroups.
+// 65 to 128 strips: the two row parts (skinny.h) make 256 of 8 staged rows.  Measured at N = 1040 .. 2048, us a call, decode kernel -> wide:
 // K = 6144 plain at 12 / 16 rows 5.64 / 5.60 -> 6.08 / 6.40, residual 6.17 / 6.19 -> 6.67 / 7.06 (K = 4096 and 5120 alike: 0.3 to 2.1
 // slower); K = 2048 with the norm 4.81 -> 5.38, with the activation 3.56 -> 3.86, residual 3.63 -> 3.88, plain the same (K = 1536: norm 0.2
 // slower, the rest within 0.2); K <= 1024 and 2560 .. 3072 0.2 to 0.6 faster, and the norm with the activation 0.6 to 1.7 everywhere.
+// Up to 64 strips: K in whole units of 128 has the half strips below (with the norm the decode kernel takes two launches: 6.9 -> 5.3).  Odd
+// chunks, N = 224 .. 1024, 9 / 16 rows: K = 3136 plain 4.7 -> 5.4 / 6.0, residual 4.9 -> 5.8 / 6.7, 6080 at 16 rows 5.8 -> 6.4, K <= 3008
+// 0.1 to 0.5 faster; the norm at 1600 / 1984 5.0 -> 5.2 / 5.4, at 1088 5.0 -> 4.9.
 // The activation alone at 3072 < K <= 4096: 1.1 to 1.9 slower on up to 64 strips too (longer K has no decode form: 0.8 to 1.4 faster).
-inline bool row_parts_keep(int64_t m, int64_t strips, int64_t k, int form) {
+inline bool decode_keeps(int64_t m, int64_t strips, int64_t k, int form) {
   if (m > 16 || strips > 128 || form == kWideNormPair) return false;
   if (form == kWidePair && k > 3072) return k <= 4096;
-  return strips > 64 && (k > 3072 || (k > 1024 && k <= 2048));
+  if (strips > 64) return k > 3072 || (k > 1024 && k <= 2048);
+  return k % 128 != 0 && form != kWidePair && k > (form == kWideNorm ? 1280 : 3072);
 }
 
 // The tile of kWideTiles for the automatic choice of an [m, k] x [n, k] call on strip weights, or -1: 9 to 128 rows (8 and
@@ -59,7 +63,7 @@ inline int wide_cfg(int64_t m, int64_t n, int64_t k, int form) {
   if ((form == kWidePlain || form == kWideFp8) && k <= 1024 && m > 48) return -1;
   if (m < (norm && k <= 1024 ? 5 : 9) || m > 128 || n <= 0 || n > (1 << 30) || k % 64 != 0 || k <= 512 || k > 6144) return -1;
   const int64_t strips = (n + 15) / 16, chunks = k / 64;
-  if (row_parts_keep(m, strips, k, form)) return -1;
+  if (decode_keeps(m, strips, k, form)) return -1;
   int waves, cpw;
   if (chunks <= 16) waves = 8, cpw = 2;
   else if (chunks <= 32) waves = strips > 128 ? 16 : 8, cpw = strips > 128 ? 2 : 4;
