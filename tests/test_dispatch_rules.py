@@ -174,3 +174,36 @@ int main() {
         else:
             want = not (3072 < k <= 4096 and m <= 16)
         assert taken == want, (k, n, m, form)
+
+
+def test_wide_grids_fill_one_round_of_each_die(tmp_path):
+    """Workgroups go to the eight dies in turn, 32 compute units each: no die gets a second round of a grid that the rule counts
+    as one, with the columns padded to eights in each row block or not."""
+    rows = _run(tmp_path, """
+#include <stdio.h>
+#include <initializer_list>
+#include "wide_rule.h"
+using namespace qtts;
+int main() {
+  int worst = 0, calls = 0, padded = 0;
+  for (int k : {768, 1024, 1536, 2048, 3072, 6144})
+    for (int n = 32; n <= 20000; n += 32)
+      for (int m = 5; m <= 128; ++m)
+        for (int form = 1; form <= 16; form *= 2) {
+          const int t = wide_cfg(m, n, k, form);
+          if (t < 0) continue;
+          const int cols = ((n + 15) / 16 + kWideTiles[t].nb - 1) / kWideTiles[t].nb, blocks = (m + 16 * kWideTiles[t].mb - 1) / (16 * kWideTiles[t].mb);
+          const int x = wide_grid_x(cols, blocks);
+          int die[8] = {0};
+          for (int b = 0; b < blocks; ++b)
+            for (int c = 0; c < cols; ++c) ++die[(b * x + c) % 8];
+          for (int d = 0; d < 8; ++d) worst = die[d] > worst ? die[d] : worst;
+          ++calls;
+          padded += x % 8 == 0;
+          if (x < cols) worst = 1000;
+        }
+  printf("%d %d %d\\n", worst, calls, padded);
+}
+""")
+    worst, calls, padded = rows[0]
+    assert worst == 32 and calls > 10000 and padded > 0.9 * calls

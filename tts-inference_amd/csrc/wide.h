@@ -368,8 +368,8 @@ struct WideArgs {
 template <typename XT, int EPI, bool NORM, bool F8W, int FORM, int I> inline void launch_wide_tile(const WideArgs& a) {
   if constexpr ((kWideTiles[I].forms & FORM) != 0) {
     constexpr WideTile t = kWideTiles[I];
-    const int64_t strips = (a.n + 15) / 16;
-    const dim3 grid((unsigned)(((strips + t.nb - 1) / t.nb + 7) / 8 * 8), 1, (unsigned)((a.m + 16 * t.mb - 1) / (16 * t.mb)));
+    const int64_t strips = (a.n + 15) / 16, blocks = (a.m + 16 * t.mb - 1) / (16 * t.mb);
+    const dim3 grid((unsigned)wide_grid_x((strips + t.nb - 1) / t.nb, blocks), 1, (unsigned)blocks);
     auto run = [&](auto fit, auto nt) {
       qtts::launch(&w8a16_wide_kernel<XT, t.mb, t.nb, t.waves, t.cpw, t.cl, EPI, NORM, F8W, decltype(nt)::value, decltype(fit)::value>,
                    grid, dim3(t.waves * 64), 0, a.st, a.qs, (const XT*)a.x, a.scale, (const XT*)a.bias, (const XT*)a.aux,

@@ -22,6 +22,22 @@ constexpr WideTile kWideTiles[] = {
     {1, 1, 16, 6, 4, 21}, {1, 2, 16, 6, 4, 21}};
 constexpr int kWideTileCount = (int)(sizeof(kWideTiles) / sizeof(kWideTiles[0]));
 
+// The grid's x for `cols` columns of tiles in `blocks` row blocks.  Workgroups go to the eight dies (32 compute units and an L2
+// each) in turn, so with x a multiple of 8 a column's row blocks meet on one die and read its weights through one L2; of 4 or 2,
+// on two or four.  The largest of these that leaves every die at most 32 of the workgroups that have a tile, else x = cols:
+// 85 columns x 3 blocks, 255 workgroups, would be 33 on five dies at x = 88 (39 rows of 5408 x 1536 with the norm: 12.8 us, 9.4 at
+// x = 85).  41 columns x 6 blocks (90 rows of 1312 x 6144) 12.0 us at x = 41, 9.9 at 42; 33 x 7 (100 of 1056 x 6144) 11.6 at 33, 8.1 at 36.
+inline int64_t wide_grid_x(int64_t cols, int64_t blocks) {
+  for (int64_t step = 8; step > 1; step /= 2) {
+    const int64_t x = (cols + step - 1) / step * step;
+    int64_t extra[8] = {0}, most = 0;
+    for (int64_t b = 0; b < blocks; ++b)
+      for (int64_t c = 0; c < cols % 8; ++c) most = most > ++extra[(b * x + c) % 8] ? most : extra[(b * x + c) % 8];
+    if (cols / 8 * blocks + most <= 32) return x;
+  }
+  return cols;
+}
+
 // Whether the decode kernel keeps a call of 9 to 16 rows on up to 128 strips, where this kernel has at most 128 workgroups.
 // 65 to 128 strips: the two row parts (skinny.h) make 256 of 8 staged rows.  Measured at N = 1040 .. 2048, us a call, decode kernel -> wide:
 // K = 6144 plain at 12 / 16 rows 5.64 / 5.60 -> 6.08 / 6.40, residual 6.17 / 6.19 -> 6.67 / 7.06 (K = 4096 and 5120 alike: 0.3 to 2.1
