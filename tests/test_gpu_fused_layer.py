@@ -343,7 +343,9 @@ WIDE = [(5, 4096, 1024), (6, 4096, 1024), (7, 6144, 1024), (8, 1024, 1024), (9, 
 # K between the tiles' full runs: waves whose runs differ by one chunk, each group of tiles at the ends of its range of K
 WIDE_K = [(5, 4096, 640), (9, 1040, 576), (16, 4096, 960), (48, 1000, 704), (17, 6144, 1088), (33, 2048, 1088), (64, 1040, 1984),
           (128, 4096, 1984), (9, 4096, 2112), (27, 1000, 2624), (97, 1024, 3008), (12, 4096, 3136), (32, 2048, 5120), (64, 2048, 6080),
-          (27, 12288, 1536)]
+          (27, 12288, 1536),
+          # grids whose row blocks are not a multiple of 8 columns apart; few strips of odd chunks, on the decode kernel
+          (39, 5408, 1536), (90, 1312, 6144), (100, 1056, 3072), (16, 544, 3136), (9, 224, 1984)]
 
 
 def _ref64(h, q, s, b):
